@@ -868,11 +868,33 @@ static int launch_linear_rows(hipStream_t stream, const void *x, int T, int in_d
   return GLM_OK;
 }
 
+bool glm_dense_gemm_supported(int T, int K, int N, int fmt, const uint8_t *s0, const uint8_t *s1);
+int glm_dense_gemm_launch(hipStream_t stream, int nproj, const uint16_t *x, int T, int K,
+                          const void *w0, const uint8_t *s0, const void *w1, const uint8_t *s1,
+                          int fmt, int N, float limit, uint16_t *out);
+
+// Whether a resident linear (nproj 1) or the two gate/up projections run as a
+// tiled GEMM (dense_gemm.hip) instead of streaming tiles: from 65 tokens on
+// (MXFP8, K = N = 4096: 20.6 against 21 us at 64 tokens, 25 against 20 at 65,
+// 63 against 21 at 200; the streaming tiles go over the weights once per 64
+// tokens), and at any count where K has no split for the streaming tiles,
+// which would leave the scalar kernel.
+static bool dense_gemm_rule(int T, int fmt, int nproj, int K, int N, const uint8_t *s0,
+                            const uint8_t *s1) {
+  constexpr int kMinT = 65;
+  int ksplit, cpw;
+  return (T >= kMinT || !choose_split(fmt, nproj, K, &ksplit, &cpw)) &&
+         glm_dense_gemm_supported(T, K, N, fmt, s0, s1);
+}
+
 int glm_linear_launch(hipStream_t stream, const uint16_t *x, int T, int in_dims,
                       const void *weight, const uint8_t *scales, int fmt, int out_dims,
                       uint16_t *y) {
   if (linear_rows_supported(T, in_dims, out_dims))
     return launch_linear_rows<false>(stream, x, T, in_dims, weight, scales, fmt, out_dims, y);
+  if (dense_gemm_rule(T, fmt, 1, in_dims, out_dims, scales, nullptr))
+    return glm_dense_gemm_launch(stream, 1, x, T, in_dims, weight, scales, nullptr, nullptr, fmt,
+                                 out_dims, 0.0f, y);
   GemvArgs a{};
   a.act = x;
   a.w[0] = a.w[1] = static_cast<const uint8_t *>(weight);
@@ -896,18 +918,23 @@ int glm_mlp_launch(hipStream_t stream, const uint16_t *x, int T, int d, int I, i
     return glm_grouped_dense_mlp_launch(stream, x, T, d, I, static_cast<const uint16_t *>(gw),
                                         static_cast<const uint16_t *>(uw),
                                         static_cast<const uint16_t *>(dw), limit, h, out);
-  GemvArgs a{};
-  a.act = x;
-  a.w[0] = static_cast<const uint8_t *>(gw);
-  a.w[1] = static_cast<const uint8_t *>(uw);
-  a.s[0] = gs;
-  a.s[1] = us;
-  a.N = I;
-  a.K = d;
-  a.dense_rows = T;
-  a.out = h;
-  a.limit = glm_limit_bf16(limit);
-  int rc = glm_gemv_launch(stream, fmt, 2, a, T > 0 ? 1 : 0);
+  int rc;
+  if (dense_gemm_rule(T, fmt, 2, d, I, gs, us)) {
+    rc = glm_dense_gemm_launch(stream, 2, x, T, d, gw, gs, uw, us, fmt, I, limit, h);
+  } else {
+    GemvArgs a{};
+    a.act = x;
+    a.w[0] = static_cast<const uint8_t *>(gw);
+    a.w[1] = static_cast<const uint8_t *>(uw);
+    a.s[0] = gs;
+    a.s[1] = us;
+    a.N = I;
+    a.K = d;
+    a.dense_rows = T;
+    a.out = h;
+    a.limit = glm_limit_bf16(limit);
+    rc = glm_gemv_launch(stream, fmt, 2, a, T > 0 ? 1 : 0);
+  }
   if (rc != GLM_OK) return rc;
   return glm_linear_launch(stream, h, T, I, dw, ds, fmt, d, out);
 }
