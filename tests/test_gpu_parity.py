@@ -132,6 +132,36 @@ def test_mx_quantize_bit_exact(gu, bits, rule):
     np.testing.assert_array_equal(gu.host(codes), want_codes)
 
 
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("rule", [O.MX_RULE_NEAREST, O.MX_RULE_OCP])
+@pytest.mark.parametrize("groups", [1, 3, 65, 6145])
+def test_mx_quantize_aligned_equals_any_alignment(gu, bits, rule, groups):
+    """The vector kernel against the one for buffers off its alignment, byte
+    for byte: every bf16 pattern (NaN, infinities, subnormals, both zeros) in
+    groups of like and of mixed magnitudes."""
+    torch = _torch()
+    rng = np.random.default_rng(groups)
+    every = np.arange(65536, dtype=np.uint16)  # consecutive patterns: one binade to a group
+    w = np.concatenate([every, rng.permutation(every), rng.permutation(every)[:2048]]).reshape(-1, 32)
+    w = np.concatenate([w, w])[rng.permutation(2 * len(w))[:groups]]
+    n = w.size * bits // 8
+    fmt = native.GLM_FMT_MXFP8 if bits == 8 else native.GLM_FMT_MXFP4
+    src = torch.empty(w.size + 8, dtype=torch.int16, device="cuda")
+    got = []
+    for off in (0, 1):  # elements of w, bytes of the codes
+        src[off:off + w.size].copy_(torch.from_numpy(w.reshape(-1).view(np.int16)))
+        codes = torch.full((n + 8,), 0xa5, dtype=torch.uint8, device="cuda")
+        scales = torch.full((groups + 8,), 0xa5, dtype=torch.uint8, device="cuda")
+        gu.call("glm_mx_quantize", gu.stream(), src[off:].data_ptr(), groups, 32, fmt, rule,
+                codes[off:].data_ptr(), scales[off:].data_ptr())
+        c, s = gu.host(codes), gu.host(scales)
+        assert np.all(c[:off] == 0xa5) and np.all(c[off + n:] == 0xa5)
+        assert np.all(s[:off] == 0xa5) and np.all(s[off + groups:] == 0xa5)
+        got.append((c[off:off + n], s[off:off + groups]))
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+
+
 # --------------------------------------------------------------------------- router / dispatch
 
 
