@@ -1141,15 +1141,17 @@ __device__ __forceinline__ void w8_body(const SplitArgs &a, long long e, int pos
 #pragma unroll
   for (int j = 0; j < kWL; ++j) {
     const int g = j * kW8Waves + wv;
-    const int feat = f0 + (NPROJ == 2 ? (16 * g) % kHalf : 16 * g);
+    // (the last feature tile may end past N: its staged rows there repeat the
+    // last ones, and the waves that own them compute and store nothing)
+    const int feat = min(f0 + (NPROJ == 2 ? (16 * g) % kHalf : 16 * g), a.N - 16);
     wuni[j] = (uint32_t)(feat / 16) * (uint32_t)(K / 128) * 1024u;
   }
   const __amdgpu_buffer_rsrc_t wsrs =
       make_rsrc(a.s[NPROJ == 2 && wv >= 4 ? 1 : 0] + e * a.s_stride,
                 (uint32_t)a.N * (uint32_t)(K / 32));
   const uint32_t wslane = (uint32_t)lane * (uint32_t)(K / 32);
-  const uint32_t wsuni =
-      (uint32_t)(f0 + (NPROJ == 2 ? (wv * 64) % kHalf : wv * 64)) * (uint32_t)(K / 32);
+  const uint32_t wsuni = (uint32_t)min(f0 + (NPROJ == 2 ? (wv * 64) % kHalf : wv * 64), a.N - 64) *
+                         (uint32_t)(K / 32);
   // every wave loads 64 scale slots (wave w: slots 64 w mod the padded
   // count, so waves past the last slot repeat earlier ones with the same
   // bytes); padding slots load slot 0's scale
@@ -1553,9 +1555,12 @@ __device__ __forceinline__ void w8_item(const SplitArgs &a, int lin) {
   // row 0 takes the odd one); blocks past the tile's rows are not computed
   const int nblk = (rows + 15) >> 4;
   const int half = 16 * ((nblk + 1) >> 1);
-  const int wt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 2;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wt = wv >> 2;
   const int tok0 = wt ? half : 0;
-  const int nb = wt ? nblk - (half >> 4) : (half >> 4);
+  int nb = wt ? nblk - (half >> 4) : (half >> 4);
+  // gate/up, N an odd multiple of 128: the last tile's waves past N load only
+  if (NPROJ == 2 && ftile * (kSplitTileW / 2) + (wv & 3) * 64 >= a.N) nb = 0;
   switch (nb) {
     case 5: w8_body<NPROJ, AF, 5>(a, tile.x, tile.y, rows, ftile, tok0); break;
     case 4: w8_body<NPROJ, AF, 4>(a, tile.x, tile.y, rows, ftile, tok0); break;
@@ -1592,10 +1597,16 @@ using namespace glm;
 int glm_grouped_tile_rows() { return kSplitTileM; }
 
 // Whether the grouped GEMMs cover these shapes: gate/up K = d, N = I in
-// feature tiles of 128 per projection; down K = I, N = d in tiles of 256.
+// feature tiles of 256 per projection; down K = I, N = d in tiles of 512.
 bool glm_grouped_supported(int d, int I) {
   return d % 512 == 0 && I % 256 == 0;
 }
+
+// The layer's grouped path (exact FP8 split) also takes an I that leaves half
+// of the last gate/up feature tile empty: at d 2560, E 120, k 6, I 896, 300
+// tokens 193 us, where the decode kernels or GEMVs over the work list are
+// what else covers it (62 ms as one thread per output).
+bool glm_grouped_layer_supported(int d, int I) { return d % 512 == 0 && I % 128 == 0; }
 
 static int grouped_launch(hipStream_t stream, GroupedArgs a, int nproj, int max_tiles) {
   // gate/up: 192-row tiles (96 features of each projection) when 256-row
@@ -1692,7 +1703,8 @@ static void launch_f8f6f4(hipStream_t stream, dim3 grid, const SplitArgs &a) {
 }
 
 static int split_launch(hipStream_t stream, SplitArgs a, int nproj, int max_tiles, int af) {
-  a.feature_tiles = a.N / (nproj == 2 ? kSplitTileW / 2 : kSplitTileW);
+  const int tile_n = nproj == 2 ? kSplitTileW / 2 : kSplitTileW;
+  a.feature_tiles = (a.N + tile_n - 1) / tile_n;
   a.max_tiles = max_tiles;
   // XCD x handles items [x * per, (x + 1) * per) with per <= ceil(max_items / 8),
   // at linear ids x + 8k: the grid must reach 8 * ceil(max_items / 8)
@@ -1828,7 +1840,7 @@ int glm_grouped_gate_up_shared_launch(hipStream_t stream, const void *x_split, i
   a.K = d;
   a.out = h;
   a.limit = glm_limit_bf16(limit);
-  a.feature_tiles = a.N / (kSplitTileW / 2);
+  a.feature_tiles = (a.N + kSplitTileW / 2 - 1) / (kSplitTileW / 2);
   const long long r_items = (long long)max_tiles * a.feature_tiles;
   const long long routed_blocks = (r_items + kXcds - 1) / kXcds * kXcds;
   GroupedArgs sh{};

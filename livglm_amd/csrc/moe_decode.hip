@@ -1020,14 +1020,25 @@ size_t glm_select_dispatch_lds_bytes(int EPL) {
 
 // Whether the decode kernels cover this layer shape: gate/up waves take d/512
 // chunks of 128 (d / 4 per wave), down waves the whole K = I in I/128 chunks
-// (16 at the real expert geometry, I 2048); the shared expert's down tiles
-// take 1 or 2 chunks per K range.
-static bool chunk_count_ok(int c) { return c == 1 || c == 2 || c == 4 || c == 6 || c == 8; }
-static bool down_chunks_ok(int c) { return chunk_count_ok(c) || c == 16; }
-static bool shared_chunks_ok(int c) { return c == 1 || (c % 2 == 0 && c <= 16); }
+// (16 at the real expert geometry, I 2048).  A wave's chunks are one batch of
+// loads whatever their count, so every count within the registers is taken;
+// a count left out puts the layer on the work-list GEMVs, or on one thread per
+// output where K has no split there: two layers of one token at d 3072, I 896
+// took 495 us (63 here), 23 tokens at d 2560, I 896 26.6 ms (94 us).
+static bool gate_up_chunks_ok(int c) { return c >= 2 && c <= 8; }
+static bool down_chunks_ok(int c) { return (c >= 1 && c <= 10) || c == 16; }
+
+// The shared expert's down tiles take K ranges of 1 to 3 chunks, at most
+// kPairMaxParts of them: pairs, else one chunk each (counts up to 7), else
+// threes (9, 15).  0: no such split.
+static int shared_range_chunks(int c) {
+  if (c % 2 == 0) return c <= 16 ? 2 : 0;
+  if (c <= 7) return 1;
+  return c % 3 == 0 && c <= 15 ? 3 : 0;
+}
 
 bool glm_decode_gate_up_supported(int d, int I) {
-  return d % 512 == 0 && d / 512 >= 2 && chunk_count_ok(d / 512) && I % 16 == 0;
+  return d % 512 == 0 && gate_up_chunks_ok(d / 512) && I % 16 == 0;
 }
 
 bool glm_decode_down_supported(int I, int d) {
@@ -1037,16 +1048,16 @@ bool glm_decode_down_supported(int I, int d) {
 bool glm_decode_path_supported(int T, int d, int E, int k, int I, int Is) {
   if (T < 1 || T > 64 || (long long)T * k > kMaxFusedPairs || E > kFusedMaxE) return false;
   // gate/up: 4 waves x CPW chunks of 128 over d; down: 64-row tiles of d
-  if (d % 512 != 0 || !chunk_count_ok(d / 512) || d / 512 < 2) return false;
+  if (d % 512 != 0 || !gate_up_chunks_ok(d / 512)) return false;
   if (I % 128 != 0 || !down_chunks_ok(I / 128)) return false;
-  if (Is > 0 && (Is % 128 != 0 || !shared_chunks_ok(Is / 128))) return false;
+  if (Is > 0 && (Is % 128 != 0 || shared_range_chunks(Is / 128) == 0)) return false;
   return true;
 }
 
 // Shared-expert splits: gate/up K in d/512 ranges when T <= 8 (one 128-wide
-// chunk per wave), else full-K tiles; down K in ranges of 2 chunks (1 if Is == 128).
+// chunk per wave), else full-K tiles; down K in ranges of shared_range_chunks.
 int glm_decode_shared_skq(int T, int d) { return T <= 8 ? d / 512 : 1; }
-int glm_decode_shared_cpws(int Is) { return Is / 128 == 1 ? 1 : 2; }
+int glm_decode_shared_cpws(int Is) { return shared_range_chunks(Is / 128); }
 int glm_decode_shared_skd(int Is) { return Is / 128 / glm_decode_shared_cpws(Is); }
 
 static SharedArgs make_shared_args(const uint16_t *x, int T, int d, const uint16_t *sg,
@@ -1082,8 +1093,11 @@ static int launch_route_logits(hipStream_t stream, const RouteArgs &a, const Sha
 #define GLM_LOGITS(TT)                                                                          \
   switch (cpw) {                                                                                \
     case 2: hipLaunchKernelGGL((route_logits_kernel<TT, 2>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
+    case 3: hipLaunchKernelGGL((route_logits_kernel<TT, 3>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
     case 4: hipLaunchKernelGGL((route_logits_kernel<TT, 4>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
+    case 5: hipLaunchKernelGGL((route_logits_kernel<TT, 5>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
     case 6: hipLaunchKernelGGL((route_logits_kernel<TT, 6>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
+    case 7: hipLaunchKernelGGL((route_logits_kernel<TT, 7>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
     default: hipLaunchKernelGGL((route_logits_kernel<TT, 8>), g1, dim3(kRouteThreads), 0, stream, a, sh); break; \
   }
   // tokens per pass over the expert's router row
@@ -1150,8 +1164,11 @@ int glm_route_decode_launch(hipStream_t stream, const uint16_t *x, int T, int d,
   }
     switch (d / 512) {
       case 2: GLM_SS(2) break;
+      case 3: GLM_SS(3) break;
       case 4: GLM_SS(4) break;
+      case 5: GLM_SS(5) break;
       case 6: GLM_SS(6) break;
+      case 7: GLM_SS(7) break;
       default: GLM_SS(8) break;
     }
 #undef GLM_SS
@@ -1173,6 +1190,8 @@ int glm_route_decode_launch(hipStream_t stream, const uint16_t *x, int T, int d,
 #define GLM_SEL(EP)                                                                           \
   if (cs == 1)                                                                                \
     hipLaunchKernelGGL((select_dispatch_kernel<EP, 1>), g2, dim3(kRouteThreads), lds, stream, a, sh); \
+  else if (cs == 3)                                                                           \
+    hipLaunchKernelGGL((select_dispatch_kernel<EP, 3>), g2, dim3(kRouteThreads), lds, stream, a, sh); \
   else                                                                                        \
     hipLaunchKernelGGL((select_dispatch_kernel<EP, 2>), g2, dim3(kRouteThreads), lds, stream, a, sh)
   if (e8 == 1) GLM_SEL(1);
@@ -1230,8 +1249,11 @@ int glm_decode_gate_up_launch(hipStream_t stream, const uint16_t *x, int T, int 
   const int blocks = a.shared_blocks + a.slots * (I / 16);
   switch (d / 512) {
     case 2: hipLaunchKernelGGL(decode_gate_up_kernel<2>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
+    case 3: hipLaunchKernelGGL(decode_gate_up_kernel<3>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
     case 4: hipLaunchKernelGGL(decode_gate_up_kernel<4>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
+    case 5: hipLaunchKernelGGL(decode_gate_up_kernel<5>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
     case 6: hipLaunchKernelGGL(decode_gate_up_kernel<6>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
+    case 7: hipLaunchKernelGGL(decode_gate_up_kernel<7>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
     case 8: hipLaunchKernelGGL(decode_gate_up_kernel<8>, dim3(blocks), dim3(256), lds, stream, a, sh); break;
     default: glm::set_error("decode gate/up: unsupported d=%d", d); return GLM_ERR_UNSUPPORTED_SHAPE;
   }
@@ -1270,14 +1292,21 @@ int glm_decode_down_launch(hipStream_t stream, const uint16_t *h, int T, int k, 
 #define GLM_DOWN(CR)                                                                            \
   if (cs == 1)                                                                                  \
     hipLaunchKernelGGL((decode_down_kernel<CR, 1>), dim3(blocks), dim3(256), lds, stream, a, sh); \
+  else if (cs == 3)                                                                             \
+    hipLaunchKernelGGL((decode_down_kernel<CR, 3>), dim3(blocks), dim3(256), lds, stream, a, sh); \
   else                                                                                          \
     hipLaunchKernelGGL((decode_down_kernel<CR, 2>), dim3(blocks), dim3(256), lds, stream, a, sh)
   switch (I / 128) {
     case 1: GLM_DOWN(1); break;
     case 2: GLM_DOWN(2); break;
+    case 3: GLM_DOWN(3); break;
     case 4: GLM_DOWN(4); break;
+    case 5: GLM_DOWN(5); break;
     case 6: GLM_DOWN(6); break;
+    case 7: GLM_DOWN(7); break;
     case 8: GLM_DOWN(8); break;
+    case 9: GLM_DOWN(9); break;
+    case 10: GLM_DOWN(10); break;
     case 16: GLM_DOWN(16); break;
     default: glm::set_error("decode down: unsupported I=%d", I); return GLM_ERR_UNSUPPORTED_SHAPE;
   }
@@ -1309,22 +1338,31 @@ static int launch_select_gate_up(hipStream_t stream, const PairArgs &a, const Sh
       std::max(pair_gate_up_lds_bytes(d, epl) + (sx ? pair_gate_up_sx_bytes(d, a.tpb) : 0),
                (size_t)T * cs * 128 * 2);
   const dim3 g2(a.routed_blocks + sh.dn_blocks);
-#define GLM_PAIR_GU_D(EP, CS, SX)                                                              \
-  switch (d / 512) {                                                                           \
-    case 2: hipLaunchKernelGGL((select_gate_up_kernel<EP, 2, CS, SX>), g2, dim3(256), lds2, stream, a, sh); break; \
-    case 4: hipLaunchKernelGGL((select_gate_up_kernel<EP, 4, CS, SX>), g2, dim3(256), lds2, stream, a, sh); break; \
-    case 6: hipLaunchKernelGGL((select_gate_up_kernel<EP, 6, CS, SX>), g2, dim3(256), lds2, stream, a, sh); break; \
-    default: hipLaunchKernelGGL((select_gate_up_kernel<EP, 8, CS, SX>), g2, dim3(256), lds2, stream, a, sh); break; \
-  }
-#define GLM_PAIR_GU(EP, CS)       \
-  if (sx) {                       \
-    GLM_PAIR_GU_D(EP, CS, true)   \
-  } else {                        \
-    GLM_PAIR_GU_D(EP, CS, false)  \
+#define GLM_PAIR_GU_C(EP, C, CS, SX)                                                          \
+  case C: hipLaunchKernelGGL((select_gate_up_kernel<EP, C, CS, SX>), g2, dim3(256), lds2, stream, a, sh); break;
+#define GLM_PAIR_GU_EVEN(EP, CS, SX) \
+  GLM_PAIR_GU_C(EP, 2, CS, SX)       \
+  GLM_PAIR_GU_C(EP, 4, CS, SX)       \
+  GLM_PAIR_GU_C(EP, 6, CS, SX)       \
+  GLM_PAIR_GU_C(EP, 8, CS, SX)
+#define GLM_PAIR_GU(EP, CS)           \
+  if (sx) {                           \
+    switch (d / 512) {                \
+      GLM_PAIR_GU_EVEN(EP, CS, true)  \
+    }                                 \
+  } else {                            \
+    switch (d / 512) {                \
+      GLM_PAIR_GU_EVEN(EP, CS, false) \
+      GLM_PAIR_GU_C(EP, 3, CS, false) \
+      GLM_PAIR_GU_C(EP, 5, CS, false) \
+      GLM_PAIR_GU_C(EP, 7, CS, false) \
+    }                                 \
   }
 #define GLM_PAIR_GU_CS(EP) \
   if (cs == 1) {           \
     GLM_PAIR_GU(EP, 1)     \
+  } else if (cs == 3) {    \
+    GLM_PAIR_GU(EP, 3)     \
   } else {                 \
     GLM_PAIR_GU(EP, 2)     \
   }
@@ -1339,7 +1377,8 @@ static int launch_select_gate_up(hipStream_t stream, const PairArgs &a, const Sh
   }
 #undef GLM_PAIR_GU_CS
 #undef GLM_PAIR_GU
-#undef GLM_PAIR_GU_D
+#undef GLM_PAIR_GU_EVEN
+#undef GLM_PAIR_GU_C
   GLM_LAUNCH_CHECK("select_gate_up_kernel");
   return GLM_OK;
 }
@@ -1347,6 +1386,14 @@ static int launch_select_gate_up(hipStream_t stream, const PairArgs &a, const Sh
 bool glm_pair_path_supported(int T, int d, int E, int k, int I, int Is) {
   return T >= 1 && T <= kPairMaxT && k <= kPairMaxK && d % 16 == 0 &&
          glm_decode_path_supported(T, d, E, k, I, Is);
+}
+
+// The shapes that the few-token kernels take with Mode-B scale rows, and that
+// the entry point of the selection with the routed gate/up takes.
+bool glm_pair_path_even_chunks(int d, int I, int Is) {
+  const int c = d / 512, ci = I / 128, cs = Is / 128;
+  return c % 2 == 0 && (ci == 1 || (ci % 2 == 0 && (ci <= 8 || ci == 16))) &&
+         (cs <= 1 || cs % 2 == 0);
 }
 
 // The three-kernel token-major layer (T <= 4): logits (+ shared gate/up),
@@ -1440,20 +1487,30 @@ int glm_pair_path_launch(hipStream_t stream, const uint16_t *x, int T, int d, co
   const size_t lds3 = (size_t)k * lds_row_stride(I) * 2 +
                       (sx ? (size_t)k * 16 * b.tpb * (I / 32) : 0);
   const dim3 g3(T * (d / 16) / b.tpb), b3(64 * std::max(k, 4));
-#define GLM_PAIR_DN(SX)                                                                      \
-  switch (I / 128) {                                                                         \
-    case 1: hipLaunchKernelGGL((down_combine_kernel<1, SX>), g3, b3, lds3, stream, b); break; \
-    case 2: hipLaunchKernelGGL((down_combine_kernel<2, SX>), g3, b3, lds3, stream, b); break; \
-    case 4: hipLaunchKernelGGL((down_combine_kernel<4, SX>), g3, b3, lds3, stream, b); break; \
-    case 6: hipLaunchKernelGGL((down_combine_kernel<6, SX>), g3, b3, lds3, stream, b); break; \
-    case 8: hipLaunchKernelGGL((down_combine_kernel<8, SX>), g3, b3, lds3, stream, b); break; \
-    default: hipLaunchKernelGGL((down_combine_kernel<16, SX>), g3, b3, lds3, stream, b); break; \
-  }
+#define GLM_PAIR_DN(C, SX) \
+  case C: hipLaunchKernelGGL((down_combine_kernel<C, SX>), g3, b3, lds3, stream, b); break;
+#define GLM_PAIR_DN_EVEN(SX) \
+  GLM_PAIR_DN(1, SX)         \
+  GLM_PAIR_DN(2, SX)         \
+  GLM_PAIR_DN(4, SX)         \
+  GLM_PAIR_DN(6, SX)         \
+  GLM_PAIR_DN(8, SX)         \
+  GLM_PAIR_DN(16, SX)
   if (sx) {
-    GLM_PAIR_DN(true)
+    switch (I / 128) {
+      GLM_PAIR_DN_EVEN(true)
+    }
   } else {
-    GLM_PAIR_DN(false)
+    switch (I / 128) {
+      GLM_PAIR_DN_EVEN(false)
+      GLM_PAIR_DN(3, false)
+      GLM_PAIR_DN(5, false)
+      GLM_PAIR_DN(7, false)
+      GLM_PAIR_DN(9, false)
+      GLM_PAIR_DN(10, false)
+    }
   }
+#undef GLM_PAIR_DN_EVEN
 #undef GLM_PAIR_DN
   GLM_LAUNCH_CHECK("down_combine_kernel");
   return GLM_OK;
@@ -1479,7 +1536,8 @@ extern "C" int glm_route_gate_up(void *stream, const float *logits, const float 
               GLM_ERR_INVALID_ARGUMENT, "route_gate_up: null pointer argument");
   GLM_REQUIRE(glm_aligned16({x, gate_packed, gate_scales, up_packed, up_scales, h}),
               GLM_ERR_INVALID_ARGUMENT, "route_gate_up: buffers must be 16-byte aligned");
-  GLM_REQUIRE(T <= kPairMaxT && top_k <= kPairMaxK && glm_pair_path_supported(T > 0 ? T : 1, d, E, top_k, I, 0),
+  GLM_REQUIRE(T <= kPairMaxT && top_k <= kPairMaxK && glm_pair_path_supported(T > 0 ? T : 1, d, E, top_k, I, 0) &&
+                  glm_pair_path_even_chunks(d, I, 0),
               GLM_ERR_UNSUPPORTED_SHAPE,
               "route_gate_up: unsupported shape T=%d d=%d E=%d k=%d I=%d (T <= 4, k <= 8, "
               "E <= 448, d/512 in {2,4,6,8}, I/128 in {1,2,4,6,8,16})",

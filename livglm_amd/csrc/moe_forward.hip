@@ -49,7 +49,7 @@ int glm_dispatch_launch(hipStream_t stream, const uint32_t *indices, int T, int 
                         int32_t *chunk_scratch);
 size_t glm_dispatch_chunk_ints(long long P, int E);
 int glm_grouped_tile_rows();
-bool glm_grouped_supported(int d, int I);
+bool glm_grouped_layer_supported(int d, int I);
 bool glm_split_fits(long long rows, int K);
 size_t glm_act_split_bytes(long long rows, int K);
 int glm_act_split_launch(hipStream_t stream, const uint16_t *x, long long rows, int K,
@@ -85,6 +85,7 @@ int glm_combine_launch(hipStream_t stream, const uint16_t *y, const int32_t *inv
                        const uint16_t *shared, int T, int k, int d, float *out);
 bool glm_decode_path_supported(int T, int d, int E, int k, int I, int Is);
 bool glm_pair_path_supported(int T, int d, int E, int k, int I, int Is);
+bool glm_pair_path_even_chunks(int d, int I, int Is);
 int glm_pair_path_launch(hipStream_t stream, const uint16_t *x, int T, int d, const float *w,
                          const float *bias, int E, int k, int n_group, int topk_group, int norm,
                          float scale, float *logits, float *weights, uint32_t *indices, int I,
@@ -465,7 +466,8 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
   const bool shared_bf16 = has_shared && shared_fmt == GLM_FMT_BF16;
   const uint16_t *shared_ready = shared_in;  // caller-computed shared output, if any
   const bool fuse_shared = shared_bf16 && !shared_in;
-  GLM_REQUIRE(!sx_rows || glm_pair_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0),
+  GLM_REQUIRE(!sx_rows || (glm_pair_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0) &&
+                           glm_pair_path_even_chunks(d, I, fuse_shared ? Is : 0)),
               GLM_ERR_UNSUPPORTED_SHAPE,
               "moe_forward_scalex: coded scales are decoded by the few-token kernels, which take "
               "T <= 4, top_k <= 8, d / 512 in {2, 4, 6, 8} and I / 128 in {1, 2, 4, 6, 8, 16} "
@@ -532,7 +534,7 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
   // mostly padding)
   // (the grouped GEMMs address the FP8 splits of x and h with 32-bit offsets:
   // beyond 4 GiB of split the layer stays on the GEMV kernels)
-  const bool grouped = glm_grouped_supported(d, I) && T > 64 && glm_split_fits(T, d) &&
+  const bool grouped = glm_grouped_layer_supported(d, I) && T > 64 && glm_split_fits(T, d) &&
                        glm_split_fits((long long)T * top_k, I);
   // with the bf16 router GEMM, x's FP8 split rides in the router weights'
   // split launch (one kernel, two block ranges)

@@ -309,7 +309,8 @@ def test_dispatch_bit_exact(gu, T, k, E, kind):
     assert got["status"][0] == 0
 
 
-@pytest.mark.parametrize("T,k,E", [(2, 2, 4), (900, 8, 32), (9000, 8, 448)])
+@pytest.mark.parametrize("T,k,E", [(2, 2, 4), (63, 1, 1), (65, 1, 448), (128, 8, 7), (205, 5, 31),
+                                   (512, 8, 448), (900, 8, 32), (9000, 8, 448)])
 def test_dispatch_flags_out_of_range(gu, T, k, E):
     # pairs with an index >= E are dropped on the one-workgroup path, the
     # chunk-parallel one with the counts in the scan's workgroup (900 x 8
@@ -890,10 +891,11 @@ SMALL_LAYERS = [
     (3, 256, 64, 64, 64, 64, (1, 1)),
     # the real expert geometry with few experts (d = 4096, I = 2048, I_shared 1024)
     (3, 4096, 24, 8, 2048, 1024, (1, 1)),
-    # shapes the decode kernels do not cover (d / 512 = 3) but the grouped GEMMs
-    # do: up to 64 tokens they run the tiled GEMV kernels over the work list with
-    # many pairs per expert (several 16-token batches, the act_index loop), from
-    # 65 tokens the grouped GEMMs -- both sides of the threshold
+    # shapes that neither the decode kernels nor the grouped GEMMs cover (d % 512):
+    # the tiled GEMV kernels over the work list with many pairs per expert
+    # (several 16-token batches, the act_index loop)
+    (40, 768, 8, 8, 256, 256, (1, 1)),
+    # both sides of the decode kernels' and the grouped GEMMs' threshold
     (40, 1536, 8, 8, 256, 256, (1, 1)),
     (64, 1536, 16, 8, 256, 256, (1, 1)),
     (65, 1536, 16, 8, 256, 256, (1, 1)),
@@ -902,6 +904,24 @@ SMALL_LAYERS = [
     # decode path (~21 pairs per expert, two 16-row h batches)
     (2, 4096, 288, 8, 2048, 2048, (1, 1)),
     (64, 4096, 24, 8, 2048, 2048, (1, 1)),
+    # every chunk count of the few-token and the decode kernels that is not a
+    # power of two or 6: gate/up 3, 5, 7 (d / 512), down 3, 5, 7, 9, 10 (I / 128),
+    # shared down ranges of 1 and 3 chunks (I_shared 384, 640, 896; 1152)
+    (1, 1536, 64, 6, 640, 640, (1, 1)),
+    (2, 2560, 40, 5, 896, 896, (1, 1)),
+    (4, 3584, 32, 4, 1152, 1152, (1, 1)),
+    (3, 1536, 24, 8, 1280, 1280, (1, 1)),
+    (7, 2560, 24, 4, 384, 384, (1, 1)),
+    (12, 3584, 16, 4, 640, 1152, (1, 1)),
+    (24, 1536, 16, 4, 1152, 640, (2, 1)),
+    (40, 2560, 16, 8, 1280, 1152, (1, 1)),
+    (64, 3584, 12, 4, 896, 384, (1, 1)),
+    # grouped GEMMs whose last gate/up feature tile is half empty, the first one
+    # too (I 128), with an odd count of K chunks in the down GEMM
+    (65, 512, 8, 2, 128, 0, (1, 1)),
+    (100, 1536, 8, 4, 384, 384, (1, 1)),
+    (300, 1024, 8, 4, 640, 640, (1, 1)),
+    (700, 512, 16, 8, 1152, 128, (1, 1)),
 ]
 
 

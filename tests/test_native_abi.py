@@ -270,6 +270,22 @@ def test_scalex_forward_rejects_short_stride_on_host(lib):
         assert "directory" in msg
 
 
+@pytest.mark.parametrize("d,I,Is", [(1536, 768, 0), (2048, 640, 0), (2048, 1280, 0), (2048, 768, 384)])
+def test_entry_points_of_even_chunk_counts_refuse_others(lib, d, I, Is):
+    # the layer takes these widths; with Mode-B scale rows (and, but for the
+    # shared expert's width, as the routed gate/up alone) they stay refused
+    fake = ctypes.c_void_p(0x1000)  # never dereferenced: validation fails first
+    rows, sh = ctypes.c_void_p(0x10000), fake if Is else None
+    msg = _expect(native.GLM_ERR_UNSUPPORTED_SHAPE, "glm_moe_forward_scalex", None, fake, 2, d,
+                  fake, fake, 128, 8, 1, 1, 1, 2.5, I, fake, fake, fake, rows, 1 << 20, Is,
+                  native.GLM_FMT_BF16, sh, None, sh, None, sh, None, None, 10.0, fake, 1 << 40,
+                  fake, None, None)
+    assert "few-token" in msg
+    if Is == 0:
+        _expect(native.GLM_ERR_UNSUPPORTED_SHAPE, "glm_route_gate_up", None, fake, fake, 2, 128, 8,
+                1, 1, 1, 2.5, fake, d, I, fake, fake, fake, fake, 10.0, fake, fake, fake)
+
+
 def test_split_beyond_32_bit_offsets_is_rejected_on_host(lib):
     # the grouped GEMMs address an activation split through 32-bit offsets: a
     # split above 4 GiB is refused instead of read as zeros past the limit
