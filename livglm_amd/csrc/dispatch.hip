@@ -59,7 +59,34 @@ __device__ __forceinline__ int2 row_tile(int c, int nt, int i) {
   return make_int2(r0, r1 - r0);
 }
 
-// Single workgroup; LDS: cnt[E] off[E] run[E] bits[E][32] + scan scratch.
+constexpr int kDispatchWaves = kDispatchThreads / 64;
+constexpr int kMaxDispatchE = 448;
+// Pairs of the single-workgroup dispatch, four to a thread.
+constexpr int kSinglePairs = 4096;
+
+// Lanes of the wave that hold this lane's key (at most E): one ballot per bit.
+__device__ __forceinline__ uint64_t same_key_lanes(uint32_t key, int E) {
+  const int nbits = 32 - __clz(E);
+  uint64_t same = ~0ull;
+  for (int bit = 0; bit < nbits; ++bit) {
+    const uint64_t m = __ballot((key >> bit) & 1u);
+    same &= ((key >> bit) & 1u) ? m : ~m;
+  }
+  return same;
+}
+__device__ __forceinline__ int lanes_below(uint64_t mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Single workgroup, P <= kSinglePairs, E <= kMaxDispatchE.  A pair's place is
+// its expert's offset + that expert's pairs in earlier groups of 64 pairs (one
+// wave's turn each) + its rank among the lanes of its own turn (as
+// dispatch_rank_kernel).  A chain of latencies: the indices, one LDS pass over
+// the turns' counts by a thread an expert, one scan.  LDS: counts, then
+// prefixes, [turns][E].  The layer at 2,664
+// pairs and 128 experts takes 157.9 us instead of 178.5 (a chunk of 1,024
+// pairs at a time through bitmaps in LDS: 29.4 us for this kernel alone).
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_kernel(
     const uint32_t *__restrict__ idx, int P, int k, int E, int32_t *__restrict__ counts,
     int32_t *__restrict__ offsets, int32_t *__restrict__ perm, int32_t *__restrict__ inv,
@@ -67,107 +94,97 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_kernel(
     int32_t *__restrict__ num_active, int4 *__restrict__ work, int32_t *__restrict__ status,
     int tile_rows, int4 *__restrict__ tiles, int32_t *__restrict__ num_tiles) {
   extern __shared__ uint32_t smem[];
-  uint32_t *cnt = smem;
-  uint32_t *off = cnt + E;
-  uint32_t *run = off + E;
-  uint32_t *bits = run + E;  // [E][32]: one bit per pair of the current 1024-pair chunk
-  __shared__ int s_scan[kDispatchThreads / 64 + 1];
+  uint16_t *turn = reinterpret_cast<uint16_t *>(smem);  // [turns][E]
+  __shared__ int s_scan[kDispatchWaves + 1];
+  __shared__ int32_t s_off[kMaxDispatchE];
   __shared__ int s_bad;
-  const int tid = threadIdx.x;
-
-  for (int e = tid; e < E; e += kDispatchThreads) {
-    cnt[e] = 0;
-    run[e] = 0;
+  constexpr int kPer = kSinglePairs / kDispatchThreads;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int turns = (P + 63) / 64;
+  uint32_t key[kPer];  // E stands for "no pair" (past the end, or an index >= E, dropped)
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int p = u * kDispatchThreads + tid;
+    key[u] = p < P ? idx[p] : (uint32_t)E;
   }
+  for (int i = tid; i < (turns * E + 1) / 2; i += kDispatchThreads) smem[i] = 0;
   if (tid == 0) s_bad = 0;
   __syncthreads();
-  for (int p = tid; p < P; p += kDispatchThreads) {
-    const uint32_t e = idx[p];
-    if (e < (uint32_t)E) atomicAdd(&cnt[e], 1u);
-    else s_bad = 1;
+  int below[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    if (u * kDispatchThreads >= P) break;  // uniform
+    if (key[u] >= (uint32_t)E) {
+      if (u * kDispatchThreads + tid < P) s_bad = 1;
+      key[u] = E;
+    }
+    const uint64_t same = same_key_lanes(key[u], E);
+    below[u] = lanes_below(same);
+    if (key[u] < (uint32_t)E && below[u] == 0)
+      turn[(u * kDispatchWaves + wave) * E + key[u]] = (uint16_t)__popcll(same);
   }
   __syncthreads();
-
-  // offsets = exclusive scan of counts; active = compacted ids with count > 0;
-  // optionally the row tiles of the grouped GEMMs (row_tile, in expert
-  // order): {expert, first sorted position, rows, 0}.
-  int carry = 0, carry_active = 0, carry_tiles = 0;
-  for (int e0 = 0; e0 < E; e0 += kDispatchThreads) {
-    const int e = e0 + tid;
-    const int c = e < E ? (int)cnt[e] : 0;
-    int tot = 0;
-    const int ex = block_exclusive_scan(c, s_scan, &tot);
-    int tot_a = 0;
-    const int ex_a = block_exclusive_scan(c > 0 ? 1 : 0, s_scan, &tot_a);
-    const int nt = tiles != nullptr ? row_tiles(c, tile_rows) : 0;
-    int tot_t = 0;
-    const int ex_t = block_exclusive_scan(nt, s_scan, &tot_t);
-    if (e < E) {
-      off[e] = carry + ex;
-      offsets[e] = carry + ex;
-      counts[e] = c;
-      if (c > 0) {
-        active[carry_active + ex_a] = e;
-        work[carry_active + ex_a] = make_int4(e, carry + ex, c, 0);
-      }
-      for (int i = 0; i < nt; ++i) {
-        const int2 t = row_tile(c, nt, i);
-        tiles[carry_tiles + ex_t + i] = make_int4(e, carry + ex + t.x, t.y, 0);
+  // expert tid: exclusive prefix over the turns, its total
+  int total = 0;
+  if (tid < E) {
+    for (int w0 = 0; w0 < turns; w0 += 8) {
+      int n[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) n[j] = w0 + j < turns ? turn[(w0 + j) * E + tid] : 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (w0 + j < turns) turn[(w0 + j) * E + tid] = (uint16_t)total;
+        total += n[j];
       }
     }
-    carry += tot;
-    carry_active += tot_a;
-    carry_tiles += tot_t;
+  }
+  // one scan for the pairs (at most 2^12), the active experts (448) and the
+  // row tiles (2^12 / 16 + 448), packed from bit 0, 13 and 22
+  const int nt = tiles != nullptr && tid < E ? row_tiles(total, tile_rows) : 0;
+  int all = 0;
+  const uint32_t ex = (uint32_t)block_exclusive_scan(
+      (int)((uint32_t)total | (total > 0 ? 1u << 13 : 0u) | (uint32_t)nt << 22), s_scan, &all);
+  const int off = ex & 0x1fff, ex_a = (ex >> 13) & 0x1ff, ex_t = ex >> 22;
+  const int pairs = all & 0x1fff, tot_a = ((uint32_t)all >> 13) & 0x1ff;
+  if (tid < E) {
+    s_off[tid] = off;
+    offsets[tid] = off;
+    counts[tid] = total;
+    if (total > 0) {
+      active[ex_a] = tid;
+      work[ex_a] = make_int4(tid, off, total, 0);
+    }
+    for (int i = 0; i < nt; ++i) {
+      const int2 t = row_tile(total, nt, i);
+      tiles[ex_t + i] = make_int4(tid, off + t.x, t.y, 0);
+    }
   }
   if (tid == 0) {
-    offsets[E] = carry;
-    num_active[0] = carry_active;
+    offsets[E] = pairs;
+    num_active[0] = tot_a;
     status[0] = s_bad;
-    if (num_tiles != nullptr) num_tiles[0] = carry_tiles;
+    if (num_tiles != nullptr) num_tiles[0] = (int)((uint32_t)all >> 22);
   }
-  for (int e = carry_active + tid; e < E; e += kDispatchThreads) {
-    active[e] = -1;
-    work[e] = make_int4(-1, 0, 0, 0);
+  for (int x = tot_a + tid; x < E; x += kDispatchThreads) {
+    active[x] = -1;
+    work[x] = make_int4(-1, 0, 0, 0);
   }
   __syncthreads();
-
-  // Stable ranks, one 1024-pair chunk at a time: rank(p) = run[e] + number
-  // of earlier pairs of this chunk with the same expert (bitmap popcount).
-  for (int p0 = 0; p0 < P; p0 += kDispatchThreads) {
-    for (int w = tid; w < E * 32; w += kDispatchThreads) bits[w] = 0;
-    __syncthreads();
-    const int p = p0 + tid;
-    uint32_t e = 0xffffffffu;
-    if (p < P) {
-      e = idx[p];
-      if (e < (uint32_t)E) atomicOr(&bits[e * 32 + (tid >> 5)], 1u << (tid & 31));
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int p = u * kDispatchThreads + tid;
+    if (p >= P) break;
+    if (key[u] < (uint32_t)E) {
+      const int pos = s_off[key[u]] + turn[(u * kDispatchWaves + wave) * E + key[u]] + below[u];
+      perm[pos] = p;
+      inv[p] = pos;
+      pair_token[pos] = p / k;
+    } else {
+      inv[p] = -1;
     }
-    __syncthreads();
-    if (p < P) {
-      if (e < (uint32_t)E) {
-        const uint32_t *row = bits + e * 32;
-        uint32_t r = run[e];
-        const int word = tid >> 5;
-        for (int w = 0; w < word; ++w) r += __popc(row[w]);
-        r += __popc(row[word] & ((1u << (tid & 31)) - 1u));
-        const int pos = (int)(off[e] + r);
-        perm[pos] = p;
-        inv[p] = pos;
-        pair_token[pos] = p / k;
-      } else {
-        inv[p] = -1;
-      }
-    }
-    __syncthreads();
-    for (int ee = tid; ee < E; ee += kDispatchThreads) {
-      uint32_t c = 0;
-      for (int w = 0; w < 32; ++w) c += __popc(bits[ee * 32 + w]);
-      run[ee] += c;
-    }
-    __syncthreads();
   }
   // positions past the valid pairs (dropped indices >= E) hold -1
-  for (int pos = carry + tid; pos < P; pos += kDispatchThreads) {
+  for (int pos = pairs + tid; pos < P; pos += kDispatchThreads) {
     perm[pos] = -1;
     pair_token[pos] = -1;
   }
@@ -187,8 +204,6 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_kernel(
 // counts, work list and row tiles.  The result is identical to the
 // single-workgroup dispatch.
 // ---------------------------------------------------------------------------
-constexpr int kDispatchWaves = kDispatchThreads / 64;
-
 // LDS: per-wave expert counts [kDispatchWaves][E] (E <= 448).
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_rank_kernel(
     const uint32_t *__restrict__ idx, int P, int E, int32_t *__restrict__ chunk_counts,
@@ -204,15 +219,8 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_rank_kernel(
   const uint32_t key = e < (uint32_t)E ? e : (uint32_t)E;
   __syncthreads();
   if (p < P && e >= (uint32_t)E) s_bad = 1;
-  // the lanes holding this lane's key: one ballot per bit of the key
-  const int nbits = 32 - __clz(E);
-  uint64_t same = ~0ull;
-  for (int bit = 0; bit < nbits; ++bit) {
-    const uint64_t m = __ballot((key >> bit) & 1u);
-    same &= ((key >> bit) & 1u) ? m : ~m;
-  }
-  const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
-                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+  const uint64_t same = same_key_lanes(key, E);
+  const int below = lanes_below(same);
   if (key < (uint32_t)E && below == 0) wcnt[wave * E + key] = __popcll(same);
   __syncthreads();
   // per expert: exclusive prefix over the waves; the chunk's count
@@ -240,7 +248,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_place_kernel(
     int32_t *__restrict__ offsets, int32_t *__restrict__ active, int32_t *__restrict__ num_active,
     int4 *__restrict__ work, int32_t *__restrict__ status, int tile_rows,
     int4 *__restrict__ tiles, int32_t *__restrict__ num_tiles) {
-  __shared__ int32_t base[448];
+  __shared__ int32_t base[kMaxDispatchE];
   __shared__ int s_scan[kDispatchThreads / 64 + 1];
   const int tid = threadIdx.x;
   const int chunk = blockIdx.x;
@@ -375,11 +383,14 @@ extern "C" int glm_moe_tiles(void *stream, const int32_t *work, int E, int32_t *
   return GLM_OK;
 }
 
-size_t glm_dispatch_lds_bytes(int E) { return (size_t)E * (3 + 32) * sizeof(uint32_t); }
+// LDS of the single-workgroup dispatch: a 16-bit count per turn and expert.
+static size_t dispatch_lds_bytes(int P, int E) {
+  return ((size_t)((P + 63) / 64) * E + 1) / 2 * sizeof(uint32_t);
+}
 
 // Pairs above which the dispatch runs on many workgroups (it then needs
 // glm_dispatch_chunk_ints(P, E) ints of scratch).
-constexpr int kMultiDispatchPairs = 4096;
+constexpr int kMultiDispatchPairs = glm::kSinglePairs;
 size_t glm_dispatch_chunk_ints(long long P, int E) {
   return P > kMultiDispatchPairs
              ? (size_t)((P + glm::kDispatchThreads - 1) / glm::kDispatchThreads) * (E + 1)
@@ -425,7 +436,7 @@ int glm_dispatch_launch(hipStream_t stream, const uint32_t *indices, int T, int 
     return GLM_OK;
   }
   hipLaunchKernelGGL(glm::dispatch_kernel, dim3(1), dim3(glm::kDispatchThreads),
-                     glm_dispatch_lds_bytes(E), stream, indices, P, k, E, counts, offsets, perm,
+                     dispatch_lds_bytes(P, E), stream, indices, P, k, E, counts, offsets, perm,
                      inv, pair_token, active, num_active, work, status, tile_rows, tiles,
                      num_tiles);
   GLM_LAUNCH_CHECK("dispatch_kernel");
