@@ -25,6 +25,18 @@ struct HcFuse {
   int hc, bf16;                    // bf16: GLM_HC_BF16_STREAMS rounding points
 };
 
+// A dense product that rides in a grouped GEMM's launch (grouped_stream.hip):
+// out [T][N] = x [T][K] W^T, or the SwiGLU of two such products (w[1], s[1] the
+// up projection), W row-major in format fmt.
+struct RidingGemm {
+  const uint16_t *x;
+  int T, K, N, fmt;
+  const void *w[2];
+  const uint8_t *s[2];
+  float limit;
+  uint16_t *out;
+};
+
 }  // namespace glm
 
 #define GLM_REQUIRE(cond, code, ...)  \

@@ -1,0 +1,456 @@
+// Block-scaled grouped GEMMs for few rows per expert, where the experts'
+// weights are what a launch waits for (the layer's routed projections,
+// native_expert_ssd.py:726-743, as grouped_gemm.hip's wide forms).
+//
+// A workgroup is four waves over a row tile of up to 64 rows x 256 weight rows
+// (gate/up: 128 features of each projection), a wave 64 weight rows x all of
+// the tile's rows.  A wave's weights are its own, so they go from the
+// tile-major bank straight into registers in the MFMA's operand order, two
+// chunks of 4 KB ahead; only the activations, which all four waves read, and
+// the scales pass through LDS (a ring of three stages, filled by direct loads
+// in the same order).  That leaves room for two workgroups a CU, whose loads
+// overlap each other's barriers, first loads and epilogues; the wide forms
+// have one workgroup a CU with a 32 KB chunk of weights in flight and nothing
+// beside its start and end.  Layers of uniform
+// routing, wide forms in brackets: d 2048, E 128, k 8, I 768, 333 tokens
+// 114 us (157); d 4096, E 288, k 8, I 2048, 66 tokens 598 us (793), 200 tokens
+// 739 us (912, gate/up at 5.2 TB/s here), 1023 tokens 915 us (1128).  More
+// stages (4) measured 1 % slower, two stages 1 to 3 %.
+//
+// The sums run as in the wide forms (K in chunks, hi before lo), so the
+// results are theirs bit for bit.
+//
+// The shared expert's dense tiles (dense_tile.h) ride in the same launches, so
+// that its MFMAs run beside the experts' weight stream: at 333 tokens (d 2048)
+// 123 us where its two products as launches of their own made it 152, at 1500
+// (E 120, d 1536) 138 and 163.
+#include <algorithm>
+
+#include "act_split.h"
+#include "dense_tile.h"
+#include "lds_stage.h"
+#include "mfma_tile.h"
+#include "topk_select.h"  // wave_lds_sync
+
+namespace glm {
+
+constexpr int kStreamRows = 64;          // rows of a row tile
+constexpr int kStreamRing = 3;           // chunks in flight or in use
+
+struct StreamLds {
+  static constexpr int kRows = kStreamRows;
+  static constexpr int kXS = kRows * 256;              // [2 terms][16 NB] scale dwords, whole waves
+  static constexpr int kXSSlots = (2 * kRows + 63) / 64 * 64;
+  static constexpr int kWS = kXS + kXSSlots * 4;       // [256 weight rows] scale dwords
+  static constexpr int kStage = kWS + 256 * 4;
+  static constexpr int kBytes = kStreamRing * kStage;
+  static constexpr int kYRow = 144;  // bytes per row of the down epilogue's staging (128 + 16)
+  static_assert(4 * 16 * kYRow <= kBytes, "the down epilogue's staging fits the ring");
+};
+
+constexpr int kStreamThreads = 256;
+constexpr int kStreamCUs = 256;
+constexpr int kStreamTileW = 256;  // weight rows per workgroup
+
+template <int N>
+struct StreamStage {
+  static constexpr int value = N;
+};
+typedef int glm_i32x8 __attribute__((ext_vector_type(8)));
+
+// A weight load; NT: non-temporal, for weights that one row tile reads.
+template <bool NT>
+__device__ __forceinline__ glm_u32x4 buf16_load(__amdgpu_buffer_rsrc_t rs, uint32_t voff,
+                                                uint32_t soff) {
+  return __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, NT ? 2 : 0);
+}
+
+template <int NPROJ, bool NT, int NB>
+__device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int pos0, int rows,
+                                            int ftile) {
+  using L = StreamLds;
+  constexpr int RING = kStreamRing;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int K = a.K;
+  const int nchunks = K / 128;
+  constexpr int kHalf = kStreamTileW / 2;
+  const int f0 = ftile * (kStreamTileW / NPROJ);
+  auto act_row = [&](int row) -> uint32_t {
+    const int pos = pos0 + (row < rows ? row : 0);  // past the end: re-read row 0
+    return (uint32_t)(a.act_index != nullptr ? a.act_index[pos] : pos);
+  };
+
+  // ---- load assignment, fixed over the K loop; every wave issues the same
+  // count per chunk: NB loads of 4 activation rows, one of 64 activation scale
+  // slots, one of 64 weight rows' scales, then its four weight blocks
+  constexpr int kLoads = NB + 2 + 4;
+  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.xhi, a.split_bytes);
+  const uint32_t lo_off = (uint32_t)(a.xlo - a.xhi);
+  uint32_t xoff[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int row = (j * 4 + wv) * 4 + (lane >> 4);
+    const int piece = (lane & 15) ^ (row & 15);
+    xoff[j] = act_row(row) * (uint32_t)K + (piece < 8 ? 0u : lo_off) + (piece & 7) * 16;
+  }
+  // scale slot s = term * 16 NB + row; slots past the last one (and the waves
+  // past them) repeat earlier ones
+  constexpr int kXSUsed = (2 * 16 * NB + 63) / 64 * 64;
+  const int xs0 = (wv * 64) % kXSUsed;
+  uint32_t xsoff;
+  {
+    const int s = xs0 + lane < 2 * 16 * NB ? xs0 + lane : 0;
+    xsoff = (uint32_t)((s >= 16 * NB ? a.xslo : a.xshi) - a.xhi) +
+            act_row(s % (16 * NB)) * (uint32_t)(K / 32);
+  }
+  const bool up = NPROJ == 2 && wv >= 2;  // whose scales this wave loads
+  const __amdgpu_buffer_rsrc_t wsrs =
+      make_rsrc(a.s[up ? NPROJ - 1 : 0] + e * a.s_stride, (uint32_t)a.N * (uint32_t)(K / 32));
+  const uint32_t wsoff =
+      (uint32_t)(f0 + (NPROJ == 2 ? wv * 64 % kHalf : wv * 64) + lane) * (uint32_t)(K / 32);
+  // the wave's four 16-row blocks: gate/up two of each projection (32
+  // features), down 64 consecutive features
+  const uint32_t wbytes = (uint32_t)a.N * (uint32_t)(K / 2);
+  const __amdgpu_buffer_rsrc_t wrs[2] = {make_rsrc(a.w[0] + e * a.w_stride, wbytes),
+                                         make_rsrc(a.w[NPROJ - 1] + e * a.w_stride, wbytes)};
+  uint32_t wuni[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    wuni[b] = (uint32_t)((f0 + (NPROJ == 2 ? wv * 32 + (b % 2) * 16 : wv * 64 + b * 16)) / 16) *
+              (uint32_t)(K / 128) * 1024u;
+
+  glm_u32x4 w[RING][4];
+  // the loads of chunk c into stage st; chunks past the last one read nothing
+  // (an offset past the buffer; in a split above 2 GiB another place of it),
+  // so that every step issues the same count
+  auto issue = [&](int c, int st) {
+    const bool in = c < nchunks;
+    const uint32_t far = in ? 0u : 0x80000000u;
+    const uint32_t cx = (in ? (uint32_t)c * 128u : 0u) + far, cs = (in ? (uint32_t)c * 4u : 0u) + far;
+    uint8_t *base = smem + st * L::kStage;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) buf16_to_lds(xrs, base + (j * 4 + wv) * 1024, xoff[j] + cx, 0);
+    buf4_to_lds(xrs, base + L::kXS + xs0 * 4, xsoff + cs, 0);
+    buf4_to_lds(wsrs, base + L::kWS + wv * 256, wsoff + cs, 0);
+    const uint32_t wl = 16u * lane + (in ? (uint32_t)c * 1024u : 0u) + far;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) w[st][b] = buf16_load<NT>(wrs[NPROJ == 2 ? b / 2 : 0], wl, wuni[b]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  glm_f32x4 acc[4][NB];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc[b][t] = glm_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // activation row 16 m + r, piece p at row * 256 + 16 (p ^ r); term t's
+  // operand is pieces 8 t + q and 8 t + 4 + q
+  const uint32_t xl = (uint32_t)(r * 256 + 16 * (q ^ r));
+  const uint32_t xsl = (uint32_t)(L::kXS + 4 * r + q);
+  const uint32_t wsl = (uint32_t)(L::kWS + 4 * ((NPROJ == 2 ? wv * 32 : wv * 64) + r) + q);
+  auto compute = [&](int st) {
+    const uint8_t *base = smem + st * L::kStage;
+    int wsc[4];
+    glm_i32x8 wa[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      wsc[b] = base[wsl + 4 * (NPROJ == 2 ? (b / 2) * kHalf + (b % 2) * 16 : b * 16)];
+      const glm_u32x4 v = w[st][b];
+      wa[b] = glm_i32x8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], 0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ct = 0; ct < NB; ++ct) {
+        const glm_u32x4 b0 =
+            *reinterpret_cast<const glm_u32x4 *>(base + (xl ^ (128u * t)) + ct * 4096);
+        const glm_u32x4 b1 =
+            *reinterpret_cast<const glm_u32x4 *>(base + (xl ^ (128u * t + 64u)) + ct * 4096);
+        const glm_i32x8 xb = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3],
+                              (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
+        const int xsc = base[xsl + 4 * (t * 16 * NB + ct * 16)];
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          acc[b][ct] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa[b], xb, acc[b][ct], 4, 0,
+                                                                        0, wsc[b], 0, xsc);
+      }
+  };
+
+  // Chunk c: wait for its loads (those of the RING - 2 chunks after it stay in
+  // flight), meet the other waves -- their loads of it have landed too, and
+  // none reads chunk c - 1 any more, whose stage takes chunk c + RING - 1.
+  // The loop takes RING chunks a turn, so that a chunk's stage is static; what
+  // is left over starts at stage 0 again and needs no more loads.
+#pragma unroll
+  for (int c = 0; c < RING - 1; ++c) issue(c, c);
+  int c0 = 0;
+  for (; c0 + RING <= nchunks; c0 += RING) {
+#pragma unroll
+    for (int u = 0; u < RING; ++u) {
+      // (fences: MFMAs moved across the barrier keep two chunks' operands alive)
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 2) * kLoads));
+      ring_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(c0 + u + RING - 1, (u + RING - 1) % RING);
+      compute(u);
+    }
+  }
+  auto left = [&](auto ut) {
+    constexpr int U = decltype(ut)::value;
+    if (U < RING - 1 && c0 + U < nchunks) {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((U < RING - 1 ? RING - 2 - U : 0) * kLoads));
+      ring_barrier();
+      compute(U);
+    }
+  };
+  left(StreamStage<0>{});
+  left(StreamStage<1>{});
+  left(StreamStage<2>{});
+  static_assert(RING <= 4, "at most three chunks are left over");
+  // no load may land in LDS that this workgroup reuses or leaves
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+
+  // ---- epilogue: lane (r, q) of block (b, ct) holds weight rows 4q..4q+3 of
+  // the block for token column r
+  if constexpr (NPROJ == 2) {
+    // h's FP8 hi/lo split, as the wide forms write it: the wave's 32 features
+    // of a token are one scale group, 8 per lane in lanes (r, q = 0..3)
+    const float lim = a.limit > 0.0f ? a.limit : __builtin_inff();
+    const SplitLayout S(a.out_rows, a.N);
+    const int g0 = f0 + wv * 32;
+#pragma unroll
+    for (int ct = 0; ct < NB; ++ct) {
+      const int row = ct * 16 + r;
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int m = 0; m < 4; m += 2) {
+          float ga = acc[i][ct][m], gb = acc[i][ct][m + 1];
+          float ua = acc[2 + i][ct][m], ub = acc[2 + i][ct][m + 1];
+          bf16_round2(ga, gb);
+          bf16_round2(ua, ub);
+          limited_swiglu2_fast(ga, gb, ua, ub, lim, v[4 * i + m], v[4 * i + m + 1]);
+        }
+      uint32_t ch[2], cl[2];
+      int bh, bl;
+      split_group_part(v, ch, cl, &bh, &bl);
+      if (row < rows) {
+        const size_t prow = (size_t)(pos0 + row);
+        uint8_t *hi = a.out_split + prow * a.N + g0;
+        uint8_t *lo = a.out_split + S.lo + prow * a.N + g0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          *reinterpret_cast<uint32_t *>(hi + i * 16 + 4 * q) = ch[i];
+          *reinterpret_cast<uint32_t *>(lo + i * 16 + 4 * q) = cl[i];
+        }
+        if (q == 0) {
+          a.out_split[S.shi + prow * (a.N / 32) + g0 / 32] = (uint8_t)bh;
+          a.out_split[S.slo + prow * (a.N / 32) + g0 / 32] = (uint8_t)bl;
+        }
+      }
+    }
+  } else {
+    // y through LDS so that every store writes whole 128-byte lines; the
+    // wave's area lies in stages that every wave is done with
+    ring_barrier();
+    uint8_t *yst = smem + wv * (16 * L::kYRow);
+    const int rr = lane >> 3, seg = lane & 7;
+#pragma unroll
+    for (int ct = 0; ct < NB; ++ct) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        uint32_t o[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) o[m] = f32_to_bf16(acc[b][ct][m]);
+        *reinterpret_cast<uint2 *>(yst + r * L::kYRow + (b * 16 + 4 * q) * 2) =
+            uint2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = ct * 16 + 8 * h + rr;
+        const glm_u32x4 v = *reinterpret_cast<const glm_u32x4 *>(yst + (8 * h + rr) * L::kYRow + 16 * seg);
+        if (row < rows)
+          *reinterpret_cast<glm_u32x4 *>(a.out + (size_t)(pos0 + row) * a.N + f0 + wv * 64 + 8 * seg) = v;
+      }
+      wave_lds_sync();
+    }
+  }
+}
+
+// The riding product's tile: 128 weight rows (gate/up: 64 features of each
+// projection) x 64 tokens, on four waves.
+constexpr int kRideKB = 78;  // LDS of a workgroup, two a CU
+template <int FMT>
+using RideLds = DenseLds<FMT, 2, 4, 1, kRideKB>;
+
+// Work items and their order as in the wide forms (a tile of more than
+// kStreamRows rows is cut there).  FMT >= 0: the riding product's workgroups
+// lie between the routed ones in groups of one per XCD, the first of every
+// `period` + 1 groups until there are no more of them.
+template <int NPROJ, int FMT, bool NT>
+__global__ __launch_bounds__(kStreamThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void grouped_stream_kernel(SplitArgs a, DenseArgs ride, int ride_groups, int period) {
+  int group = blockIdx.x / kXcds;
+  const int xcd = blockIdx.x % kXcds;
+  if constexpr (FMT >= 0) {
+    if (group < ride_groups * (period + 1)) {
+      const int before = group / (period + 1);
+      if (group % (period + 1) == 0)
+        return dense_item<FMT, NPROJ, 2, 4, 1, kRideKB>(ride, before * kXcds + xcd);
+      group -= before + 1;
+    } else {
+      group -= ride_groups;
+    }
+  }
+  const int nft = a.feature_tiles;
+  const int ntiles = max(0, min(*a.num_tiles, a.max_tiles));
+  const int items = ntiles * nft;
+  const int per_xcd = (items + kXcds - 1) / kXcds;
+  const int item = xcd * per_xcd + group;
+  if (group >= per_xcd || item >= items) return;
+  const int4 tile = a.tiles[item / nft];
+  if (tile.z <= 0 || tile.x < 0 || tile.y < 0) return;
+  const int rows = min(tile.z, kStreamRows);
+  const int ftile = item % nft;
+  const int nb = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
+  if (nb == 4) return stream_body<NPROJ, NT, 4>(a, tile.x, tile.y, rows, ftile);
+  if (nb == 3) return stream_body<NPROJ, NT, 3>(a, tile.x, tile.y, rows, ftile);
+  if (nb == 2) return stream_body<NPROJ, NT, 2>(a, tile.x, tile.y, rows, ftile);
+  stream_body<NPROJ, NT, 1>(a, tile.x, tile.y, rows, ftile);
+}
+
+}  // namespace glm
+
+using namespace glm;
+
+int glm_grouped_tile_rows();
+
+// Rows per tile of the layer's grouped GEMMs: the streaming form's up to 88
+// rows an expert (layer at 75 rows, d 1536, E 120, I 640: 140 against 159 us;
+// at 94, d 2048, E 128, I 768: 216 against 211) and while the wide forms'
+// tiles (256 features by at most glm_grouped_tile_rows rows) are fewer than the
+// CUs (E 16, I 512, 250 rows: 70 against 90 us, 500 rows: 97 against 101).
+int glm_grouped_layer_tile_rows(long long pairs, int E, int I) {
+  const int wide = glm_grouped_tile_rows();
+  const long long wide_items = std::max((long long)E, pairs / wide) * ((I + 255) / 256);
+  return pairs <= 88LL * E || wide_items < kStreamCUs ? kStreamRows : wide;
+}
+
+template <int NPROJ, int FMT, bool NT>
+static void launch_stream(hipStream_t stream, const SplitArgs &a, long long groups, int E,
+                          const RidingGemm *ride) {
+  DenseArgs d{};
+  long long ride_groups = 0, period = 0;
+  size_t lds = StreamLds::kBytes;
+  if constexpr (FMT >= 0) {
+    using L = RideLds<FMT>;
+    constexpr int feat = L::kRows / NPROJ;
+    d.x = ride->x;
+    for (int p = 0; p < 2; ++p) {
+      d.w[p] = static_cast<const uint8_t *>(ride->w[p]);
+      d.s[p] = ride->s[p];
+    }
+    d.out = ride->out;
+    d.T = ride->T;
+    d.N = ride->N;
+    d.K = ride->K;
+    d.limit = glm_limit_bf16(ride->limit);
+    d.row_tiles = (d.N + feat - 1) / feat;
+    d.tok_tiles = (d.T + L::kTok - 1) / L::kTok;
+    d.rows_outer = 1;
+    ride_groups = ((long long)d.row_tiles * d.tok_tiles + kXcds - 1) / kXcds;
+    // spread over the groups that have work if every expert has a tile, but for
+    // the last two rounds of the CUs: a riding item started there would end late
+    constexpr long long kRound = 2 * kStreamCUs / kXcds;
+    const long long busy = std::min(groups, ((long long)E * a.feature_tiles + kXcds - 1) / kXcds);
+    period = std::max(0LL, busy - 2 * kRound) / ride_groups;
+    lds = std::max(lds, (size_t)L::kBytes);
+  }
+  const dim3 grid((unsigned)((groups + ride_groups) * kXcds));
+  hipLaunchKernelGGL((grouped_stream_kernel<NPROJ, FMT, NT>), grid, dim3(kStreamThreads), lds, stream,
+                     a, d, (int)ride_groups, (int)period);
+}
+
+template <int NPROJ, bool NT>
+static void launch_stream_fmt(hipStream_t stream, const SplitArgs &a, long long groups, int E,
+                              const RidingGemm *ride) {
+  if (ride == nullptr)
+    launch_stream<NPROJ, -1, NT>(stream, a, groups, E, nullptr);
+  else if (ride->fmt == GLM_FMT_MXFP8)
+    launch_stream<NPROJ, FMT_MXFP8, NT>(stream, a, groups, E, ride);
+  else if (ride->fmt == GLM_FMT_MXFP4)
+    launch_stream<NPROJ, FMT_MXFP4, NT>(stream, a, groups, E, ride);
+  else
+    launch_stream<NPROJ, FMT_BF16, NT>(stream, a, groups, E, ride);
+}
+
+template <int NPROJ>
+static int stream_launch(hipStream_t stream, SplitArgs a, long long pairs, int max_tiles, int E,
+                         const RidingGemm *ride) {
+  a.feature_tiles = a.N / (kStreamTileW / NPROJ);
+  a.max_tiles = max_tiles;
+  const long long groups = ((long long)max_tiles * a.feature_tiles + kXcds - 1) / kXcds;
+  // about one row tile an expert: non-temporal weight loads (layer at 333 tokens,
+  // d 2048: 114 instead of 123 us; with two tiles an expert, 1500 tokens, 222
+  // instead of 211)
+  if (pairs <= 48LL * E)
+    launch_stream_fmt<NPROJ, true>(stream, a, groups, E, ride);
+  else
+    launch_stream_fmt<NPROJ, false>(stream, a, groups, E, ride);
+  GLM_LAUNCH_CHECK("grouped_stream_kernel");
+  return GLM_OK;
+}
+
+// The routed gate/up over row tiles of glm_grouped_layer_tile_rows rows: x's
+// split in, h's split out; `ride` (or null) a SwiGLU of two dense products.
+int glm_grouped_stream_gate_up_launch(hipStream_t stream, const void *x_split, int T,
+                                      const int32_t *pair_token, const int4 *tiles,
+                                      const int32_t *num_tiles, int max_tiles, int d, int I, int E,
+                                      const uint8_t *gw, const uint8_t *gs, const uint8_t *uw,
+                                      const uint8_t *us, float limit, void *h_split, long long P,
+                                      const RidingGemm *ride) {
+  SplitArgs a{};
+  set_split(a, x_split, T, d, ACT_FP8X2);
+  a.out_split = static_cast<uint8_t *>(h_split);
+  a.out_rows = P;
+  a.act_index = pair_token;
+  a.tiles = tiles;
+  a.num_tiles = num_tiles;
+  a.w[0] = gw;
+  a.w[1] = uw;
+  a.s[0] = gs;
+  a.s[1] = us;
+  a.w_stride = (long long)I * (d / 2);
+  a.s_stride = (long long)I * (d / 32);
+  a.N = I;
+  a.K = d;
+  a.limit = glm_limit_bf16(limit);
+  return stream_launch<2>(stream, a, P, max_tiles, E, ride);
+}
+
+// The routed down over the same tiles; `ride` (or null) one dense product.
+int glm_grouped_stream_down_launch(hipStream_t stream, const void *h_split, long long P,
+                                   const int4 *tiles, const int32_t *num_tiles, int max_tiles,
+                                   int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
+                                   uint16_t *y, const RidingGemm *ride) {
+  SplitArgs a{};
+  set_split(a, h_split, P, I, ACT_FP8X2);
+  a.tiles = tiles;
+  a.num_tiles = num_tiles;
+  a.w[0] = a.w[1] = dw;
+  a.s[0] = a.s[1] = ds;
+  a.w_stride = (long long)d * (I / 2);
+  a.s_stride = (long long)d * (I / 32);
+  a.N = d;
+  a.K = I;
+  a.out = y;
+  return stream_launch<1>(stream, a, P, max_tiles, E, ride);
+}

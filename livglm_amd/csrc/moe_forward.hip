@@ -49,6 +49,7 @@ int glm_dispatch_launch(hipStream_t stream, const uint32_t *indices, int T, int 
                         int32_t *chunk_scratch);
 size_t glm_dispatch_chunk_ints(long long P, int E);
 int glm_grouped_tile_rows();
+int glm_grouped_layer_tile_rows(long long pairs, int E, int I);
 bool glm_grouped_layer_supported(int d, int I);
 bool glm_split_fits(long long rows, int K);
 size_t glm_act_split_bytes(long long rows, int K);
@@ -63,6 +64,17 @@ int glm_grouped_gate_up_launch(hipStream_t stream, const void *x_split, int T,
 int glm_grouped_down_launch(hipStream_t stream, const void *h_split, long long P,
                             const int4 *tiles, const int32_t *num_tiles, int max_tiles, int I,
                             int d, const uint8_t *dw, const uint8_t *ds, uint16_t *y);
+int glm_grouped_stream_gate_up_launch(hipStream_t stream, const void *x_split, int T,
+                                      const int32_t *pair_token, const int4 *tiles,
+                                      const int32_t *num_tiles, int max_tiles, int d, int I, int E,
+                                      const uint8_t *gw, const uint8_t *gs, const uint8_t *uw,
+                                      const uint8_t *us, float limit, void *h_split, long long P,
+                                      const glm::RidingGemm *ride);
+int glm_grouped_stream_down_launch(hipStream_t stream, const void *h_split, long long P,
+                                   const int4 *tiles, const int32_t *num_tiles, int max_tiles,
+                                   int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
+                                   uint16_t *y, const glm::RidingGemm *ride);
+bool glm_dense_gemm_supported(int T, int K, int N, int fmt, const uint8_t *s0, const uint8_t *s1);
 int glm_gate_up_launch(hipStream_t stream, const uint16_t *x, int T, int d, int I, int E, int k,
                        const uint8_t *gw, const uint8_t *gs, const uint8_t *uw, const uint8_t *us,
                        const int32_t *pair_token, const int4 *work, float limit, uint16_t *h);
@@ -547,34 +559,64 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
                          topk_group, norm_topk_prob, routed_scaling_factor, w.logits, wts, idx,
                          w.router_split, split_early);
   if (rc) return rc;
+  const long long P = (long long)T * top_k;
+  const int tile_rows = grouped ? glm_grouped_layer_tile_rows(P, E, I) : 0;
+  const bool wide = tile_rows == glm_grouped_tile_rows();
+  int4 *tiles = w.tiles;
+  int max_tiles = w.max_tiles;
+  if (grouped && !wide) {
+    // more, smaller tiles than the workspace's list holds: they go where the
+    // logits were, which nothing reads after the selection (16 bytes a tile,
+    // at most P / 32 + E + 1 of them, against 4 T E bytes, T > 64)
+    tiles = reinterpret_cast<int4 *>(w.logits);
+    max_tiles = (int)((P + tile_rows - 1) / tile_rows) + E;
+  }
   rc = glm_dispatch_launch(stream, idx, T, top_k, E, w.counts, w.offsets, w.perm, w.inv,
-                           w.pair_token, w.active, w.num_active, w.work, w.status,
-                           grouped ? glm_grouped_tile_rows() : 0, grouped ? w.tiles : nullptr,
-                           grouped ? w.num_tiles : nullptr, w.chunk_counts);
+                           w.pair_token, w.active, w.num_active, w.work, w.status, tile_rows,
+                           grouped ? tiles : nullptr, grouped ? w.num_tiles : nullptr,
+                           w.chunk_counts);
   if (rc) return rc;
   bool shared_fused = false;
-  if (grouped) {
-    if (!split_early) {
-      rc = glm_act_split_launch(stream, x, T, d, w.x_split);
-      if (rc) return rc;
-    }
+  if (grouped && !split_early) {
+    rc = glm_act_split_launch(stream, x, T, d, w.x_split);
+    if (rc) return rc;
+  }
+  if (grouped && !wide) {
+    // the shared expert's products ride in the routed launches
+    const glm::RidingGemm gate_up{x, T, d, Is, shared_fmt, {shared_gate, shared_up},
+                                  {shared_gate_scales, shared_up_scales}, swiglu_limit, w.shared_h};
+    const glm::RidingGemm down{w.shared_h, T, Is, d, shared_fmt, {shared_down, shared_down},
+                               {shared_down_scales, shared_down_scales}, 0.0f, w.shared_out};
+    const bool ride =
+        has_shared && !shared_in &&
+        glm_dense_gemm_supported(T, d, Is, shared_fmt, shared_gate_scales, shared_up_scales) &&
+        glm_dense_gemm_supported(T, Is, d, shared_fmt, shared_down_scales, nullptr);
+    rc = glm_grouped_stream_gate_up_launch(stream, w.x_split, T, w.pair_token, tiles, w.num_tiles,
+                                           max_tiles, d, I, E, gate_packed, gate_scales, up_packed,
+                                           up_scales, swiglu_limit, w.h_split, P,
+                                           ride ? &gate_up : nullptr);
+    if (rc) return rc;  // the gate/up epilogue writes h's FP8 split for the down GEMM
+    rc = glm_grouped_stream_down_launch(stream, w.h_split, P, tiles, w.num_tiles, max_tiles, I, d,
+                                        E, down_packed, down_scales, w.y, ride ? &down : nullptr);
+    if (ride) shared_ready = w.shared_out;
+  } else if (grouped) {
     // a bf16 shared expert on the dense GEMMs: its gate/up tiles ride in the
-    // routed gate/up launch (after the routed work items)
+    // wide routed gate/up launch (after the routed work items)
     shared_fused = has_shared && !shared_in &&
                    glm_grouped_dense_mlp_supported(T, d, I_shared, shared_fmt);
     if (shared_fused)
       rc = glm_grouped_gate_up_shared_launch(
-          stream, w.x_split, T, w.pair_token, w.tiles, w.num_tiles, w.max_tiles, d, I,
+          stream, w.x_split, T, w.pair_token, tiles, w.num_tiles, max_tiles, d, I,
           gate_packed, gate_scales, up_packed, up_scales, w.h, swiglu_limit, w.h_split,
-          (long long)T * top_k, x, I_shared, static_cast<const uint16_t *>(shared_gate),
+          P, x, I_shared, static_cast<const uint16_t *>(shared_gate),
           static_cast<const uint16_t *>(shared_up), w.shared_h);
     else
-      rc = glm_grouped_gate_up_launch(stream, w.x_split, T, w.pair_token, w.tiles, w.num_tiles,
-                                      w.max_tiles, d, I, gate_packed, gate_scales, up_packed,
-                                      up_scales, w.h, swiglu_limit, w.h_split, (long long)T * top_k);
-    if (rc) return rc;  // the gate/up epilogue writes h's FP8 split for the down GEMM
-    rc = glm_grouped_down_launch(stream, w.h_split, (long long)T * top_k, w.tiles, w.num_tiles,
-                                 w.max_tiles, I, d, down_packed, down_scales, w.y);
+      rc = glm_grouped_gate_up_launch(stream, w.x_split, T, w.pair_token, tiles, w.num_tiles,
+                                      max_tiles, d, I, gate_packed, gate_scales, up_packed,
+                                      up_scales, w.h, swiglu_limit, w.h_split, P);
+    if (rc) return rc;
+    rc = glm_grouped_down_launch(stream, w.h_split, P, tiles, w.num_tiles, max_tiles, I, d,
+                                 down_packed, down_scales, w.y);
   } else {
     rc = glm_gate_up_launch(stream, x, T, d, I, E, top_k, gate_packed, gate_scales, up_packed,
                             up_scales, w.pair_token, w.work, swiglu_limit, w.h);
@@ -582,7 +624,7 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
     rc = glm_down_launch(stream, w.h, T, top_k, I, d, E, down_packed, down_scales, w.work, w.y);
   }
   if (rc) return rc;
-  if (has_shared && !shared_in) {
+  if (has_shared && shared_ready == nullptr) {
     if (shared_fused)
       rc = glm_grouped_dense_down_launch(stream, w.shared_h, T, I_shared, d,
                                          static_cast<const uint16_t *>(shared_down), w.shared_out);
