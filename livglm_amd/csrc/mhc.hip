@@ -118,6 +118,102 @@ __global__ __launch_bounds__(kHcThreads) void hc_mix_kernel(const float *x, cons
   }
 }
 
+// The same sums for many tokens on f32 MFMA: a workgroup takes 16 tokens (grid.y)
+// and one of S equal ranges of K (grid.x), its eight waves an eighth of that
+// range each; NT 16-row tiles of fn.  MFMA i of a 32-wide K step takes
+// K = k0 + 8 q + i in lane (r, q)'s slot, so a lane loads 32 contiguous bytes of
+// its token's row and of its fn rows per step; each of the eight MFMAs has
+// accumulators of its own, these and the waves' sums are added in pairs, and
+// the squares in 64 bits, which keeps the error at hc_mix_kernel's.  fn is read
+// once per 16 tokens (L2) and lanes meet once per range: hc_mix_kernel's four
+// tokens a workgroup make 24 wave sums a chunk of 256 columns, which bound it.
+// Bound by the streams' one pass: the FFN site at 1500 tokens, d 2048 takes
+// 278 us instead of 345 (one box), 333 tokens 140 instead of 156.
+constexpr int kHcMfmaWaves = 8;
+constexpr int kHcMfmaMinT = 16;
+
+template <int NT>
+__global__ __launch_bounds__(64 * kHcMfmaWaves) void hc_mix_mfma_kernel(const float *x,
+                                                                       const float *fn, int T, int K,
+                                                                       int M, float *partial) {
+  __shared__ glm_f32x4 red[kHcMfmaWaves - 1][NT][64];
+  __shared__ double rsq[kHcMfmaWaves][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int t0 = blockIdx.y * 16, s = blockIdx.x;
+  const int kw = K / ((int)gridDim.x * kHcMfmaWaves);  // a multiple of 32
+  const int kb = (s * kHcMfmaWaves + wave) * kw + 8 * q;
+  // rows past the last token or fn row repeat it (never stored)
+  const float *xr = x + (size_t)min(t0 + r, T - 1) * K + kb;
+  const float *wr[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) wr[n] = fn + (size_t)min(16 * n + r, M - 1) * K + kb;
+  glm_f32x4 acc[NT][8];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[n][i] = glm_f32x4{0.f, 0.f, 0.f, 0.f};
+  double sq2[2] = {};
+  glm_f32x4 xv[2], wv[NT][2];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xv[h] = *reinterpret_cast<const glm_f32x4 *>(xr + k + 4 * h);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) wv[n][h] = *reinterpret_cast<const glm_f32x4 *>(wr[n] + k + 4 * h);
+    }
+  };
+  load(0);
+  for (int k = 0; k < kw; k += 32) {
+    const glm_f32x4 cx[2] = {xv[0], xv[1]};
+    glm_f32x4 cw[NT][2];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      cw[n][0] = wv[n][0];
+      cw[n][1] = wv[n][1];
+    }
+    load(min(k + 32, kw - 32));  // the next step's operands fly beside these MFMAs
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float xf = cx[i / 4][i % 4];
+      sq2[i & 1] = __builtin_fma((double)xf, (double)xf, sq2[i & 1]);
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        acc[n][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xf, cw[n][i / 4][i % 4], acc[n][i],
+                                                             0, 0, 0);
+    }
+  }
+  double sq = sq2[0] + sq2[1];
+  sq += __shfl_xor(sq, 16);
+  sq += __shfl_xor(sq, 32);
+  if (q == 0) rsq[wave][r] = sq;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    acc[n][0] = ((acc[n][0] + acc[n][1]) + (acc[n][2] + acc[n][3])) +
+                ((acc[n][4] + acc[n][5]) + (acc[n][6] + acc[n][7]));
+    if (wave > 0) red[wave - 1][n][lane] = acc[n][0];
+  }
+  lds_sync();
+  if (wave != 0) return;
+  float *out = partial + ((size_t)s * T + t0) * (M + 1);
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+#pragma unroll
+    for (int w = 1; w < 4; ++w) acc[n][w] = red[2 * w - 1][n][lane] + red[2 * w][n][lane];
+    acc[n][0] = (acc[n][0] + red[0][n][lane]) + acc[n][1] + (acc[n][2] + acc[n][3]);
+    // lane (r, q) holds tokens 4q .. 4q+3 for fn row 16 n + r
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      if (t0 + 4 * q + m < T && 16 * n + r < M) out[(4 * q + m) * (M + 1) + 16 * n + r] = acc[n][0][m];
+  }
+  if (lane < 16 && t0 + lane < T) {
+    double total = 0.0;
+#pragma unroll
+    for (int w = 0; w < kHcMfmaWaves; ++w) total += rsq[w][lane];
+    out[lane * (M + 1) + M] = (float)total;
+  }
+}
+
 // A gate logit as the reference forms it: (mixed * inv_rms) * scale + base
 // (mhc.py:38-41).
 __device__ __forceinline__ float gate_logit(float raw, float inv, float scale, float base) {
@@ -389,6 +485,19 @@ static int hc_slices(int hc, int d) {
   return std::min(kHcMaxSlices, (hc * d + kHcSlice - 1) / kHcSlice);
 }
 
+// K ranges of hc_mix_mfma_kernel, or 0 where hc_mix_kernel runs: too few
+// tokens, or K not in whole steps of the eight waves.  As many ranges as bring
+// the grid to two workgroups a CU (at most hc_slices, for which the workspace
+// is sized).  From one whole token tile on: the site at 20 tokens takes 88.6 us
+// instead of 92.7.
+static int hc_mfma_slices(int T, int hc, int d) {
+  const int step = 32 * kHcMfmaWaves, K = hc * d;
+  if (T < kHcMfmaMinT || K % step != 0) return 0;
+  int S = 1;
+  while (S < 16 && (T + 15) / 16 * S < 512 && K % (2 * S * step) == 0 && 2 * S <= hc_slices(hc, d)) S *= 2;
+  return S;
+}
+
 static int check_hc(const char *who, int T, int hc, int d) {
   GLM_REQUIRE(T >= 0 && hc >= 1 && d >= 1, GLM_ERR_INVALID_ARGUMENT, "%s: invalid sizes", who);
   GLM_REQUIRE(hc <= kHcMaxMult, GLM_ERR_UNSUPPORTED_SHAPE, "%s: hc_mult %d > %d", who, hc,
@@ -430,11 +539,26 @@ extern "C" int glm_hc_pre(void *stream, const float *streams, int T, int hc, int
               glm_hc_workspace_bytes(T, hc, d));
   if (T == 0) return GLM_OK;
   const int M = 2 * hc + hc * hc;
-  const int S = hc_slices(hc, d);
+  int S = hc_slices(hc, d);
   float *partial = static_cast<float *>(workspace);
   const dim3 mix_grid(S, (T + kHcTokens - 1) / kHcTokens);
   const int rows = (M + 3) / 4;  // fn rows per wave
-  if (rows <= 2)
+  const int mfma_slices = hc_mfma_slices(T, hc, d);
+  if (mfma_slices > 0) {
+    S = mfma_slices;
+    const dim3 grid(S, (T + 15) / 16), block(64 * kHcMfmaWaves);
+#define GLM_MIX(NT)                                                                            \
+  hipLaunchKernelGGL(hc_mix_mfma_kernel<NT>, grid, block, 0, (hipStream_t)stream, streams, fn, \
+                     T, hc * d, M, partial)
+    switch ((M + 15) / 16) {
+      case 1: GLM_MIX(1); break;
+      case 2: GLM_MIX(2); break;
+      case 3: GLM_MIX(3); break;
+      case 4: GLM_MIX(4); break;
+      default: GLM_MIX(5); break;
+    }
+#undef GLM_MIX
+  } else if (rows <= 2)
     hipLaunchKernelGGL(hc_mix_kernel<2>, mix_grid, dim3(kHcThreads), 0, (hipStream_t)stream,
                        streams, fn, T, hc * d, M, partial);
   else if (rows <= 6)

@@ -64,6 +64,13 @@ def _hc_pre(gu, h, hc, d, iters, *, norm=True, bf16=False, rms_eps=1e-6, hc_eps=
     # hc = 3: the mixing-matrix sums through LDS (hc not a power of two);
     # hc d = 32768: 128 column chunks over 64 workgroups
     (2, 3, 512, 4, False), (3, 8, 4096, 6, False),
+    # from 16 tokens on f32 MFMA: partial token tiles, every count of fn row
+    # tiles (hc 1, 2 / 4 / 5, 6 / 7 / 8), one to many K ranges and steps; K off its
+    # steps (hc d = 640) stays on the other kernel
+    (16, 4, 2048, 20, False), (17, 4, 1536, 20, True), (33, 2, 128, 3, False),
+    (40, 1, 256, 1, False), (20, 6, 256, 4, False), (31, 5, 512, 4, False), (16, 7, 512, 4, False),
+    (47, 8, 1024, 5, False), (64, 4, 4096, 20, False), (300, 4, 512, 20, False),
+    (18, 2, 320, 3, False),
 ])
 def test_hc_pre_matches_oracle(gu, T, hc, d, iters, bf16):
     print(f"hc_pre T={T} hc={hc} d={d} iters={iters} bf16={bf16}", flush=True)
