@@ -11,19 +11,24 @@
 // in the same order).  That leaves room for two workgroups a CU, whose loads
 // overlap each other's barriers, first loads and epilogues; the wide forms
 // have one workgroup a CU with a 32 KB chunk of weights in flight and nothing
-// beside its start and end.  Layers of uniform
-// routing, wide forms in brackets: d 2048, E 128, k 8, I 768, 333 tokens
-// 114 us (157); d 4096, E 288, k 8, I 2048, 66 tokens 598 us (793), 200 tokens
-// 739 us (912, gate/up at 5.2 TB/s here), 1023 tokens 915 us (1128).  More
-// stages (4) measured 1 % slower, two stages 1 to 3 %.
+// beside its start and end.
 //
-// The sums run as in the wide forms (K in chunks, hi before lo), so the
-// results are theirs bit for bit.
+// Two kinds of activations.  BF: bf16 as they are, the weights converted to
+// bf16 (exact) on their way into the MFMA, which the wait for the weights
+// covers; their loads are non-temporal (about one row tile an expert).  Else
+// the wide forms' FP8 hi/lo split, twice the rows per MFMA time, in their
+// order of sums, so that the results are theirs bit for bit.
+//
+// Layers of uniform routing, the wide forms in brackets: d 2048, E 128, k 8,
+// I 768, 333 tokens 111 us (157); d 4096, E 288, k 8, I 2048, 66 tokens 586 us
+// (793), 200 tokens 703 us (912), 1023 tokens 890 us (1128).  In split form
+// without non-temporal loads 333 tokens took 123 us, with them 114; four stages
+// measured 1 % slower, two stages 1 to 3 %.
 //
 // The shared expert's dense tiles (dense_tile.h) ride in the same launches, so
-// that its MFMAs run beside the experts' weight stream: at 333 tokens (d 2048)
-// 123 us where its two products as launches of their own made it 152, at 1500
-// (E 120, d 1536) 138 and 163.
+// that its MFMAs run beside the experts' weight stream: at 333 tokens (d 2048,
+// split form) 123 us where its two products as launches of their own made it
+// 152, at 1500 (E 120, d 1536) 138 and 163.
 #include <algorithm>
 
 #include "act_split.h"
@@ -58,14 +63,14 @@ struct StreamStage {
 };
 typedef int glm_i32x8 __attribute__((ext_vector_type(8)));
 
-// A weight load; NT: non-temporal, for weights that one row tile reads.
+// A weight load; NT: non-temporal.
 template <bool NT>
 __device__ __forceinline__ glm_u32x4 buf16_load(__amdgpu_buffer_rsrc_t rs, uint32_t voff,
                                                 uint32_t soff) {
   return __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, NT ? 2 : 0);
 }
 
-template <int NPROJ, bool NT, int NB>
+template <int NPROJ, bool BF, int NB>
 __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int pos0, int rows,
                                             int ftile) {
   using L = StreamLds;
@@ -86,7 +91,8 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
   // ---- load assignment, fixed over the K loop; every wave issues the same
   // count per chunk: NB loads of 4 activation rows, one of 64 activation scale
   // slots, one of 64 weight rows' scales, then its four weight blocks
-  constexpr int kLoads = NB + 2 + 4;
+  // (BF has no activation scales)
+  constexpr int kLoads = NB + (BF ? 1 : 2) + 4;
   const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.xhi, a.split_bytes);
   const uint32_t lo_off = (uint32_t)(a.xlo - a.xhi);
   uint32_t xoff[NB];
@@ -94,14 +100,15 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
   for (int j = 0; j < NB; ++j) {
     const int row = (j * 4 + wv) * 4 + (lane >> 4);
     const int piece = (lane & 15) ^ (row & 15);
-    xoff[j] = act_row(row) * (uint32_t)K + (piece < 8 ? 0u : lo_off) + (piece & 7) * 16;
+    xoff[j] = BF ? act_row(row) * (uint32_t)(2 * K) + piece * 16
+                 : act_row(row) * (uint32_t)K + (piece < 8 ? 0u : lo_off) + (piece & 7) * 16;
   }
   // scale slot s = term * 16 NB + row; slots past the last one (and the waves
   // past them) repeat earlier ones
   constexpr int kXSUsed = (2 * 16 * NB + 63) / 64 * 64;
   const int xs0 = (wv * 64) % kXSUsed;
-  uint32_t xsoff;
-  {
+  uint32_t xsoff = 0;
+  if constexpr (!BF) {
     const int s = xs0 + lane < 2 * 16 * NB ? xs0 + lane : 0;
     xsoff = (uint32_t)((s >= 16 * NB ? a.xslo : a.xshi) - a.xhi) +
             act_row(s % (16 * NB)) * (uint32_t)(K / 32);
@@ -129,15 +136,15 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
   auto issue = [&](int c, int st) {
     const bool in = c < nchunks;
     const uint32_t far = in ? 0u : 0x80000000u;
-    const uint32_t cx = (in ? (uint32_t)c * 128u : 0u) + far, cs = (in ? (uint32_t)c * 4u : 0u) + far;
+    const uint32_t cx = (in ? (uint32_t)c * (BF ? 256u : 128u) : 0u) + far, cs = (in ? (uint32_t)c * 4u : 0u) + far;
     uint8_t *base = smem + st * L::kStage;
 #pragma unroll
     for (int j = 0; j < NB; ++j) buf16_to_lds(xrs, base + (j * 4 + wv) * 1024, xoff[j] + cx, 0);
-    buf4_to_lds(xrs, base + L::kXS + xs0 * 4, xsoff + cs, 0);
+    if constexpr (!BF) buf4_to_lds(xrs, base + L::kXS + xs0 * 4, xsoff + cs, 0);
     buf4_to_lds(wsrs, base + L::kWS + wv * 256, wsoff + cs, 0);
     const uint32_t wl = 16u * lane + (in ? (uint32_t)c * 1024u : 0u) + far;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) w[st][b] = buf16_load<NT>(wrs[NPROJ == 2 ? b / 2 : 0], wl, wuni[b]);
+    for (int b = 0; b < 4; ++b) w[st][b] = buf16_load<BF>(wrs[NPROJ == 2 ? b / 2 : 0], wl, wuni[b]);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -155,10 +162,32 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
   auto compute = [&](int st) {
     const uint8_t *base = smem + st * L::kStage;
     int wsc[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      wsc[b] = base[wsl + 4 * (NPROJ == 2 ? (b / 2) * kHalf + (b % 2) * 16 : b * 16)];
+    if constexpr (BF) {
+      // MFMA i takes K = 32 q + 8 i + s in lane (r, q): piece 4 q + i
+      float sc[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) sc[b] = e8m0_to_f32((uint32_t)wsc[b]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        glm_bf16x8 af[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) af[b] = mxfp4_word_to_bf16x8(w[st][b][i], sc[b]);
+#pragma unroll
+        for (int ct = 0; ct < NB; ++ct) {
+          const glm_bf16x8 xb = *reinterpret_cast<const glm_bf16x8 *>(
+              base + r * 256 + 16 * ((4 * q + i) ^ r) + ct * 4096);
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            acc[b][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b], xb, acc[b][ct], 0, 0, 0);
+        }
+      }
+    } else {
     glm_i32x8 wa[4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      wsc[b] = base[wsl + 4 * (NPROJ == 2 ? (b / 2) * kHalf + (b % 2) * 16 : b * 16)];
       const glm_u32x4 v = w[st][b];
       wa[b] = glm_i32x8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], 0, 0, 0, 0};
     }
@@ -178,6 +207,7 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
           acc[b][ct] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa[b], xb, acc[b][ct], 4, 0,
                                                                         0, wsc[b], 0, xsc);
       }
+    }
   };
 
   // Chunk c: wait for its loads (those of the RING - 2 chunks after it stay in
@@ -218,7 +248,22 @@ __device__ __forceinline__ void stream_body(const SplitArgs &a, long long e, int
 
   // ---- epilogue: lane (r, q) of block (b, ct) holds weight rows 4q..4q+3 of
   // the block for token column r
-  if constexpr (NPROJ == 2) {
+  if constexpr (NPROJ == 2 && BF) {
+#pragma unroll
+    for (int ct = 0; ct < NB; ++ct) {
+      const int row = ct * 16 + r;
+      if (row >= rows) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint32_t o[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          o[m] = f32_to_bf16(limited_swiglu(bf16_round(acc[i][ct][m]), bf16_round(acc[2 + i][ct][m]),
+                                            a.limit));
+        store_rows4(a.out + (size_t)(pos0 + row) * a.N + f0 + wv * 32 + i * 16 + 4 * q, o);
+      }
+    }
+  } else if constexpr (NPROJ == 2) {
     // h's FP8 hi/lo split, as the wide forms write it: the wave's 32 features
     // of a token are one scale group, 8 per lane in lanes (r, q = 0..3)
     const float lim = a.limit > 0.0f ? a.limit : __builtin_inff();
@@ -295,7 +340,7 @@ using RideLds = DenseLds<FMT, 2, 4, 1, kRideKB>;
 // kStreamRows rows is cut there).  FMT >= 0: the riding product's workgroups
 // lie between the routed ones in groups of one per XCD, the first of every
 // `period` + 1 groups until there are no more of them.
-template <int NPROJ, int FMT, bool NT>
+template <int NPROJ, bool BF, int FMT>
 __global__ __launch_bounds__(kStreamThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void grouped_stream_kernel(SplitArgs a, DenseArgs ride, int ride_groups, int period) {
   int group = blockIdx.x / kXcds;
@@ -321,10 +366,10 @@ void grouped_stream_kernel(SplitArgs a, DenseArgs ride, int ride_groups, int per
   const int rows = min(tile.z, kStreamRows);
   const int ftile = item % nft;
   const int nb = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
-  if (nb == 4) return stream_body<NPROJ, NT, 4>(a, tile.x, tile.y, rows, ftile);
-  if (nb == 3) return stream_body<NPROJ, NT, 3>(a, tile.x, tile.y, rows, ftile);
-  if (nb == 2) return stream_body<NPROJ, NT, 2>(a, tile.x, tile.y, rows, ftile);
-  stream_body<NPROJ, NT, 1>(a, tile.x, tile.y, rows, ftile);
+  if (nb == 4) return stream_body<NPROJ, BF, 4>(a, tile.x, tile.y, rows, ftile);
+  if (nb == 3) return stream_body<NPROJ, BF, 3>(a, tile.x, tile.y, rows, ftile);
+  if (nb == 2) return stream_body<NPROJ, BF, 2>(a, tile.x, tile.y, rows, ftile);
+  stream_body<NPROJ, BF, 1>(a, tile.x, tile.y, rows, ftile);
 }
 
 }  // namespace glm
@@ -332,6 +377,13 @@ void grouped_stream_kernel(SplitArgs a, DenseArgs ride, int ride_groups, int per
 using namespace glm;
 
 int glm_grouped_tile_rows();
+
+int glm_grouped_stream_rows() { return kStreamRows; }
+
+// Whether the streaming form takes bf16 activations or their split: up to 48
+// rows an expert (d 4096, E 288: 600 / 1023 tokens, 17 / 28 rows, 801 / 890
+// against 845 / 918 us; E 128, 44 rows 150 and 149; E 120, 75 rows 141 and 139).
+bool glm_grouped_stream_bf16(long long pairs, int E) { return pairs <= 48LL * E; }
 
 // Rows per tile of the layer's grouped GEMMs: the streaming form's up to 88
 // rows an expert (layer at 75 rows, d 1536, E 120, I 640: 140 against 159 us;
@@ -344,7 +396,7 @@ int glm_grouped_layer_tile_rows(long long pairs, int E, int I) {
   return pairs <= 88LL * E || wide_items < kStreamCUs ? kStreamRows : wide;
 }
 
-template <int NPROJ, int FMT, bool NT>
+template <int NPROJ, bool BF, int FMT>
 static void launch_stream(hipStream_t stream, const SplitArgs &a, long long groups, int E,
                           const RidingGemm *ride) {
   DenseArgs d{};
@@ -375,36 +427,24 @@ static void launch_stream(hipStream_t stream, const SplitArgs &a, long long grou
     lds = std::max(lds, (size_t)L::kBytes);
   }
   const dim3 grid((unsigned)((groups + ride_groups) * kXcds));
-  hipLaunchKernelGGL((grouped_stream_kernel<NPROJ, FMT, NT>), grid, dim3(kStreamThreads), lds, stream,
+  hipLaunchKernelGGL((grouped_stream_kernel<NPROJ, BF, FMT>), grid, dim3(kStreamThreads), lds, stream,
                      a, d, (int)ride_groups, (int)period);
 }
 
-template <int NPROJ, bool NT>
-static void launch_stream_fmt(hipStream_t stream, const SplitArgs &a, long long groups, int E,
-                              const RidingGemm *ride) {
-  if (ride == nullptr)
-    launch_stream<NPROJ, -1, NT>(stream, a, groups, E, nullptr);
-  else if (ride->fmt == GLM_FMT_MXFP8)
-    launch_stream<NPROJ, FMT_MXFP8, NT>(stream, a, groups, E, ride);
-  else if (ride->fmt == GLM_FMT_MXFP4)
-    launch_stream<NPROJ, FMT_MXFP4, NT>(stream, a, groups, E, ride);
-  else
-    launch_stream<NPROJ, FMT_BF16, NT>(stream, a, groups, E, ride);
-}
-
-template <int NPROJ>
-static int stream_launch(hipStream_t stream, SplitArgs a, long long pairs, int max_tiles, int E,
+template <int NPROJ, bool BF>
+static int stream_launch(hipStream_t stream, SplitArgs a, int max_tiles, int E,
                          const RidingGemm *ride) {
   a.feature_tiles = a.N / (kStreamTileW / NPROJ);
   a.max_tiles = max_tiles;
   const long long groups = ((long long)max_tiles * a.feature_tiles + kXcds - 1) / kXcds;
-  // about one row tile an expert: non-temporal weight loads (layer at 333 tokens,
-  // d 2048: 114 instead of 123 us; with two tiles an expert, 1500 tokens, 222
-  // instead of 211)
-  if (pairs <= 48LL * E)
-    launch_stream_fmt<NPROJ, true>(stream, a, groups, E, ride);
+  if (ride == nullptr)
+    launch_stream<NPROJ, BF, -1>(stream, a, groups, E, nullptr);
+  else if (ride->fmt == GLM_FMT_MXFP8)
+    launch_stream<NPROJ, BF, FMT_MXFP8>(stream, a, groups, E, ride);
+  else if (ride->fmt == GLM_FMT_MXFP4)
+    launch_stream<NPROJ, BF, FMT_MXFP4>(stream, a, groups, E, ride);
   else
-    launch_stream_fmt<NPROJ, false>(stream, a, groups, E, ride);
+    launch_stream<NPROJ, BF, FMT_BF16>(stream, a, groups, E, ride);
   GLM_LAUNCH_CHECK("grouped_stream_kernel");
   return GLM_OK;
 }
@@ -433,7 +473,7 @@ int glm_grouped_stream_gate_up_launch(hipStream_t stream, const void *x_split, i
   a.N = I;
   a.K = d;
   a.limit = glm_limit_bf16(limit);
-  return stream_launch<2>(stream, a, P, max_tiles, E, ride);
+  return stream_launch<2, false>(stream, a, max_tiles, E, ride);
 }
 
 // The routed down over the same tiles; `ride` (or null) one dense product.
@@ -452,5 +492,66 @@ int glm_grouped_stream_down_launch(hipStream_t stream, const void *h_split, long
   a.N = d;
   a.K = I;
   a.out = y;
-  return stream_launch<1>(stream, a, P, max_tiles, E, ride);
+  return stream_launch<1, false>(stream, a, max_tiles, E, ride);
+}
+
+// The same on bf16 activations: x [T][d] in, h [P][I] out.
+int glm_grouped_stream_gate_up_bf16_launch(hipStream_t stream, const uint16_t *x, int T,
+                                           const int32_t *pair_token, const int4 *tiles,
+                                           const int32_t *num_tiles, int max_tiles, int d, int I,
+                                           int E, const uint8_t *gw, const uint8_t *gs,
+                                           const uint8_t *uw, const uint8_t *us, float limit,
+                                           uint16_t *h, const RidingGemm *ride) {
+  SplitArgs a{};
+  a.xhi = a.xlo = a.xshi = a.xslo = reinterpret_cast<const uint8_t *>(x);
+  a.split_bytes = (uint32_t)((size_t)T * d * 2);
+  a.act_index = pair_token;
+  a.tiles = tiles;
+  a.num_tiles = num_tiles;
+  a.w[0] = gw;
+  a.w[1] = uw;
+  a.s[0] = gs;
+  a.s[1] = us;
+  a.w_stride = (long long)I * (d / 2);
+  a.s_stride = (long long)I * (d / 32);
+  a.N = I;
+  a.K = d;
+  a.out = h;
+  a.limit = glm_limit_bf16(limit);
+  return stream_launch<2, true>(stream, a, max_tiles, E, ride);
+}
+
+// h [P][I] in, y [P][d] out.
+int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, long long P,
+                                        const int4 *tiles, const int32_t *num_tiles, int max_tiles,
+                                        int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
+                                        uint16_t *y, const RidingGemm *ride) {
+  SplitArgs a{};
+  a.xhi = a.xlo = a.xshi = a.xslo = reinterpret_cast<const uint8_t *>(h);
+  a.split_bytes = (uint32_t)((size_t)P * I * 2);
+  a.tiles = tiles;
+  a.num_tiles = num_tiles;
+  a.w[0] = a.w[1] = dw;
+  a.s[0] = a.s[1] = ds;
+  a.w_stride = (long long)d * (I / 2);
+  a.s_stride = (long long)d * (I / 32);
+  a.N = d;
+  a.K = I;
+  a.out = y;
+  return stream_launch<1, true>(stream, a, max_tiles, E, ride);
+}
+
+// Whether the decode layer (16 to 64 tokens, the router's logits on MFMA) runs
+// on the streaming form instead of the decode kernels, which go over K in one
+// round of loads a workgroup and run an MX shared expert by itself.  At d 4096,
+// E 288, k 8, I 2048: 16 / 24 / 32 / 64 tokens 298 / 383 / 432 / 573 us (decode
+// kernels 301 / 409 / 498 / 723); d 2048, E 128, I 768: 63.9 / 74.6 / 76.1 / 86.9
+// (64.3 / 75.3 / 79.8 / 91.5), with an MXFP8 shared expert 63.6 / 74.5 / 75.9 /
+// 86.5 (74.2 / 87.4 / 93.9 / 110.8).  A layer of a few MB is launches either way
+// (d 1024, E 16, I 512: 33.3 and 32.8) and stays but for the MX shared expert's
+// own launches (33.2 and 39.0).
+bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt) {
+  if (T < 16 || T > kStreamRows || d % 512 != 0 || I % 128 != 0) return false;
+  const double weights = 1.5 * std::min((long long)E, (long long)T * k) * d * I;
+  return weights >= 32e6 || (Is > 0 && shared_fmt != GLM_FMT_BF16);
 }

@@ -50,6 +50,8 @@ int glm_dispatch_launch(hipStream_t stream, const uint32_t *indices, int T, int 
 size_t glm_dispatch_chunk_ints(long long P, int E);
 int glm_grouped_tile_rows();
 int glm_grouped_layer_tile_rows(long long pairs, int E, int I);
+int glm_grouped_stream_rows();
+bool glm_grouped_stream_bf16(long long pairs, int E);
 bool glm_grouped_layer_supported(int d, int I);
 bool glm_split_fits(long long rows, int K);
 size_t glm_act_split_bytes(long long rows, int K);
@@ -74,6 +76,17 @@ int glm_grouped_stream_down_launch(hipStream_t stream, const void *h_split, long
                                    const int4 *tiles, const int32_t *num_tiles, int max_tiles,
                                    int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
                                    uint16_t *y, const glm::RidingGemm *ride);
+int glm_grouped_stream_gate_up_bf16_launch(hipStream_t stream, const uint16_t *x, int T,
+                                           const int32_t *pair_token, const int4 *tiles,
+                                           const int32_t *num_tiles, int max_tiles, int d, int I,
+                                           int E, const uint8_t *gw, const uint8_t *gs,
+                                           const uint8_t *uw, const uint8_t *us, float limit,
+                                           uint16_t *h, const glm::RidingGemm *ride);
+int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, long long P,
+                                        const int4 *tiles, const int32_t *num_tiles, int max_tiles,
+                                        int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
+                                        uint16_t *y, const glm::RidingGemm *ride);
+bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt);
 bool glm_dense_gemm_supported(int T, int K, int N, int fmt, const uint8_t *s0, const uint8_t *s1);
 int glm_gate_up_launch(hipStream_t stream, const uint16_t *x, int T, int d, int I, int E, int k,
                        const uint8_t *gw, const uint8_t *gs, const uint8_t *uw, const uint8_t *us,
@@ -505,7 +518,9 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
     *hc_done = hc != nullptr;  // fused into the down + combine kernel
     return rc;
   }
-  if (glm_decode_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0)) {
+  const bool stream_decode = glm_grouped_stream_decode(
+      T, d, E, top_k, I, has_shared && !shared_in ? Is : 0, shared_fmt);
+  if (!stream_decode && glm_decode_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0)) {
     // decode: six short kernels, no host synchronisation; the bf16 shared
     // expert rides in the two routing kernels, or from 16 tokens on (router
     // logits on MFMA) in the two routed expert kernels
@@ -548,9 +563,17 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
   // beyond 4 GiB of split the layer stays on the GEMV kernels)
   const bool grouped = glm_grouped_layer_supported(d, I) && T > 64 && glm_split_fits(T, d) &&
                        glm_split_fits((long long)T * top_k, I);
+  const long long P = (long long)T * top_k;
+  const int tile_rows = grouped         ? glm_grouped_layer_tile_rows(P, E, I)
+                        : stream_decode ? glm_grouped_stream_rows()
+                                        : 0;
+  const bool wide = tile_rows == glm_grouped_tile_rows();
+  const bool stream_path = stream_decode || (grouped && !wide);
+  const bool stream_bf16 = stream_decode || (stream_path && glm_grouped_stream_bf16(P, E));
   // with the bf16 router GEMM, x's FP8 split rides in the router weights'
   // split launch (one kernel, two block ranges)
-  const bool split_early = grouped && w.router_split != nullptr && glm_router_split_supported(T, d);
+  const bool split_x = grouped && !stream_bf16;
+  const bool split_early = split_x && w.router_split != nullptr && glm_router_split_supported(T, d);
   if (split_early) {
     rc = glm_prefill_split_launch(stream, router_weight, E, d, w.router_split, x, T, w.x_split);
     if (rc) return rc;
@@ -559,29 +582,26 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
                          topk_group, norm_topk_prob, routed_scaling_factor, w.logits, wts, idx,
                          w.router_split, split_early);
   if (rc) return rc;
-  const long long P = (long long)T * top_k;
-  const int tile_rows = grouped ? glm_grouped_layer_tile_rows(P, E, I) : 0;
-  const bool wide = tile_rows == glm_grouped_tile_rows();
   int4 *tiles = w.tiles;
   int max_tiles = w.max_tiles;
-  if (grouped && !wide) {
+  if (stream_path) {
     // more, smaller tiles than the workspace's list holds: they go where the
     // logits were, which nothing reads after the selection (16 bytes a tile,
-    // at most P / 32 + E + 1 of them, against 4 T E bytes, T > 64)
+    // at most P / 64 + E + 1 of them, against 4 T E bytes, T >= 16)
     tiles = reinterpret_cast<int4 *>(w.logits);
     max_tiles = (int)((P + tile_rows - 1) / tile_rows) + E;
   }
   rc = glm_dispatch_launch(stream, idx, T, top_k, E, w.counts, w.offsets, w.perm, w.inv,
                            w.pair_token, w.active, w.num_active, w.work, w.status, tile_rows,
-                           grouped ? tiles : nullptr, grouped ? w.num_tiles : nullptr,
+                           tile_rows ? tiles : nullptr, tile_rows ? w.num_tiles : nullptr,
                            w.chunk_counts);
   if (rc) return rc;
   bool shared_fused = false;
-  if (grouped && !split_early) {
+  if (split_x && !split_early) {
     rc = glm_act_split_launch(stream, x, T, d, w.x_split);
     if (rc) return rc;
   }
-  if (grouped && !wide) {
+  if (stream_path) {
     // the shared expert's products ride in the routed launches
     const glm::RidingGemm gate_up{x, T, d, Is, shared_fmt, {shared_gate, shared_up},
                                   {shared_gate_scales, shared_up_scales}, swiglu_limit, w.shared_h};
@@ -591,13 +611,23 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
         has_shared && !shared_in &&
         glm_dense_gemm_supported(T, d, Is, shared_fmt, shared_gate_scales, shared_up_scales) &&
         glm_dense_gemm_supported(T, Is, d, shared_fmt, shared_down_scales, nullptr);
-    rc = glm_grouped_stream_gate_up_launch(stream, w.x_split, T, w.pair_token, tiles, w.num_tiles,
-                                           max_tiles, d, I, E, gate_packed, gate_scales, up_packed,
-                                           up_scales, swiglu_limit, w.h_split, P,
-                                           ride ? &gate_up : nullptr);
-    if (rc) return rc;  // the gate/up epilogue writes h's FP8 split for the down GEMM
-    rc = glm_grouped_stream_down_launch(stream, w.h_split, P, tiles, w.num_tiles, max_tiles, I, d,
-                                        E, down_packed, down_scales, w.y, ride ? &down : nullptr);
+    const glm::RidingGemm *ride_gu = ride ? &gate_up : nullptr, *ride_dn = ride ? &down : nullptr;
+    if (stream_bf16) {
+      rc = glm_grouped_stream_gate_up_bf16_launch(
+          stream, x, T, w.pair_token, tiles, w.num_tiles, max_tiles, d, I, E, gate_packed,
+          gate_scales, up_packed, up_scales, swiglu_limit, w.h, ride_gu);
+      if (rc) return rc;
+      rc = glm_grouped_stream_down_bf16_launch(stream, w.h, P, tiles, w.num_tiles, max_tiles, I, d,
+                                               E, down_packed, down_scales, w.y, ride_dn);
+    } else {
+      rc = glm_grouped_stream_gate_up_launch(stream, w.x_split, T, w.pair_token, tiles, w.num_tiles,
+                                             max_tiles, d, I, E, gate_packed, gate_scales,
+                                             up_packed, up_scales, swiglu_limit, w.h_split, P,
+                                             ride_gu);
+      if (rc) return rc;  // the gate/up epilogue writes h's FP8 split for the down GEMM
+      rc = glm_grouped_stream_down_launch(stream, w.h_split, P, tiles, w.num_tiles, max_tiles, I, d,
+                                          E, down_packed, down_scales, w.y, ride_dn);
+    }
     if (ride) shared_ready = w.shared_out;
   } else if (grouped) {
     // a bf16 shared expert on the dense GEMMs: its gate/up tiles ride in the

@@ -47,29 +47,41 @@ def _routed_layer(d, I, Is, k):
     return layer, shape
 
 
+def _shared_weights(layer, fmt):
+    """The shared expert's f32 matrices in format fmt (None: no shared expert),
+    its codes and scales put into the layer."""
+    if fmt is None:
+        return None
+    shared = []
+    for key in ("shared.gate", "shared.up", "shared.down"):
+        if fmt == native.GLM_FMT_BF16:
+            shared.append(O.bf16_bits_to_f32(layer[key]))
+            continue
+        bits, deq = (8, O.dequant_mxfp8) if fmt == native.GLM_FMT_MXFP8 else (4, O.dequant_mxfp4)
+        layer[key], layer[key + ".scales"] = O.quantize_mx(layer[key], bits, O.MX_RULE_NEAREST)
+        shared.append(deq(layer[key], layer[key + ".scales"]))
+    return tuple(shared)
+
+
+def _oracle(layer, shape, shared):
+    return O.moe_layer(O.bf16_bits_to_f32(layer["x"]), layer["router_weight"], layer["router_bias"],
+                       O.Bank(*(layer[key] for key in BANK_KEYS)), shared, top_k=shape.k, n_group=1,
+                       topk_group=1, norm_topk_prob=True,
+                       routed_scaling_factor=shape.routed_scaling_factor,
+                       swiglu_limit=shape.swiglu_limit, return_intermediates=True)
+
+
 @pytest.mark.parametrize("fmt", [None, native.GLM_FMT_BF16, native.GLM_FMT_MXFP8, native.GLM_FMT_MXFP4])
 @pytest.mark.parametrize("d,I,Is,k", [
-    (512, 128, 128, 1), (1024, 256, 384, 2), (1536, 384, 640, 1), (1024, 640, 160, 2),
-    (512, 512, 1280, 1),
+    # 41 rows an expert on average: bf16 activations
+    (512, 128, 128, 1), (1536, 384, 640, 1), (512, 512, 1280, 1), (1024, 640, 160, 1),
+    # 82: their FP8 split
+    (1024, 256, 384, 2), (1024, 640, 160, 2), (512, 128, 128, 2), (1536, 384, 640, 2),
 ])
 def test_stream_layer_row_and_chunk_edges(gu, d, I, Is, k, fmt):
     layer, shape = _routed_layer(d, I, Is, k)
-    shared = None
-    if fmt is not None:
-        shared = []
-        for key in ("shared.gate", "shared.up", "shared.down"):
-            if fmt == native.GLM_FMT_BF16:
-                shared.append(O.bf16_bits_to_f32(layer[key]))
-                continue
-            bits, deq = (8, O.dequant_mxfp8) if fmt == native.GLM_FMT_MXFP8 else (4, O.dequant_mxfp4)
-            layer[key], layer[key + ".scales"] = O.quantize_mx(layer[key], bits, O.MX_RULE_NEAREST)
-            shared.append(deq(layer[key], layer[key + ".scales"]))
-    want, inter = O.moe_layer(O.bf16_bits_to_f32(layer["x"]), layer["router_weight"],
-                              layer["router_bias"], O.Bank(*(layer[key] for key in BANK_KEYS)),
-                              shared and tuple(shared), top_k=k, n_group=1, topk_group=1,
-                              norm_topk_prob=True,
-                              routed_scaling_factor=shape.routed_scaling_factor,
-                              swiglu_limit=shape.swiglu_limit, return_intermediates=True)
+    shared = _shared_weights(layer, fmt)
+    want, inter = _oracle(layer, shape, shared)
     counts = np.bincount(inter["indices"].reshape(-1).astype(np.int64), minlength=shape.E)
     assert k > 1 or tuple(counts) == COUNTS
     out, w, idx = gu.run_layer(gu.upload_layer(layer), shape, shared=fmt is not None,
@@ -80,6 +92,26 @@ def test_stream_layer_row_and_chunk_edges(gu, d, I, Is, k, fmt):
     # no row of any tile is off on its own
     rows = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert rows.max() < 5 * REL_L2
+
+
+@pytest.mark.parametrize("T,d,E,k,I,Is,fmt", [
+    # decode batches: the smallest and largest of its range, an expert with a
+    # row of every token (64 in a tile), few bytes but an MX shared expert, no
+    # shared expert, one that cannot ride (I_shared 96)
+    (16, 1024, 64, 8, 512, 512, native.GLM_FMT_MXFP8), (64, 2048, 32, 8, 768, 768, native.GLM_FMT_BF16),
+    (64, 1024, 8, 8, 1280, 128, native.GLM_FMT_MXFP4), (33, 512, 16, 2, 128, 128, native.GLM_FMT_MXFP8),
+    (17, 2560, 48, 6, 640, 0, None), (40, 2048, 24, 8, 1024, 96, native.GLM_FMT_BF16),
+])
+def test_stream_decode_batches(gu, T, d, E, k, I, Is, fmt):
+    shape = MoEShape("decode", T, d, E, k, I, Is)
+    layer = make_layer(shape, 7300 + T + d)
+    shared = _shared_weights(layer, fmt)
+    want, inter = _oracle(layer, shape, shared)
+    out, w, idx = gu.run_layer(gu.upload_layer(layer), shape, shared=fmt is not None,
+                               shared_fmt=native.GLM_FMT_BF16 if fmt is None else fmt)
+    same = np.all(gu.host(idx).astype(np.uint32) == inter["indices"], axis=1)
+    assert same.sum() >= T - 1  # at most one near-tie
+    assert O.rel_l2(gu.host(out)[same], want[same]) < REL_L2
 
 
 def test_stream_gemms_equal_the_wide_forms(gu):
