@@ -147,7 +147,9 @@ def check(name: str, code: int) -> None:
 
 def call(name: str, *args) -> None:
     """Invoke ``name`` with ``args`` and raise NativeError on a non-zero status."""
-    check(name, getattr(load(), name)(*args))
+    code = getattr(_lib or load(), name)(*args)
+    if code != GLM_OK:
+        check(name, code)
 
 
 def mxfp4_is_tiled(rows: int, K: int) -> bool:

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import os
 import sys
+from functools import lru_cache
 
 import torch
 
@@ -25,7 +26,9 @@ FORMAT_OF_MODE = {None: FMT_BF16, "mxfp8": FMT_MXFP8, "mxfp4": FMT_MXFP4}
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(t.device), without building a
+    # Stream object for it (about 1 us a call)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -36,7 +39,7 @@ def require_device(t: torch.Tensor, name: str, dtypes=None) -> torch.Tensor:
     """Checks that ``t`` is a contiguous CUDA (HIP) tensor of an allowed dtype."""
     if not isinstance(t, torch.Tensor):
         raise ContractError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ContractError(f"{name} must live on the GPU (got {t.device})")
     if dtypes is not None and t.dtype not in dtypes:
         raise ContractError(f"{name} has dtype {t.dtype}, expected one of {dtypes}")
@@ -56,5 +59,6 @@ def call(name: str, *args) -> None:
         raise
 
 
+@lru_cache(maxsize=256)  # a function of the sizes alone
 def workspace_bytes(T: int, d: int, E: int, k: int, I: int, I_shared: int) -> int:
     return int(native.load().glm_moe_workspace_bytes(T, d, E, k, I, I_shared))

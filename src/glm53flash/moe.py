@@ -41,7 +41,7 @@ class TopKRouter:
             raise ContractError("router weight and bias must be float32")
         N.require_device(w, "router.weight")
         N.require_device(b, "router.e_score_correction_bias")
-        if tuple(w.shape) != (self.num_experts, self.hidden_dim) or b.numel() != self.num_experts:
+        if w.shape != (self.num_experts, self.hidden_dim) or b.numel() != self.num_experts:
             raise ContractError(f"router weight {tuple(w.shape)} / bias {tuple(b.shape)} do not "
                                 f"match E={self.num_experts}, d={self.hidden_dim}")
         return w, b
@@ -118,7 +118,9 @@ class ExpertSSDMoE:
         d = self.hidden_size
         original_shape = hidden_states.shape
         N.require_device(hidden_states, "hidden_states", (torch.bfloat16,))
-        rows = hidden_states.reshape(-1, d)
+        rows = hidden_states
+        if len(original_shape) != 2 or original_shape[1] != d:
+            rows = hidden_states.reshape(-1, d)
         T = rows.shape[0]
         dev = rows.device
         rw, rb = self.gate._params()
@@ -168,7 +170,9 @@ class ExpertSSDMoE:
                weights.data_ptr(), indices.data_ptr(), *hc_args)
         self.last_weights = weights
         self.last_indices = indices
-        return out.reshape(original_shape) if hc is None else hc_out
+        if hc is not None:
+            return hc_out
+        return out if rows is hidden_states else out.reshape(original_shape)
 
     @property
     def last_route(self) -> tuple[int, ...]:
