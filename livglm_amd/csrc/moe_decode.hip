@@ -1,4 +1,5 @@
-// Decode-size routed-MoE layer (T <= 64, T*k <= 512 pairs) in five kernels:
+// Decode-size routed-MoE layer (T <= 64, T*k <= 512 pairs; from 16 tokens on
+// only small layers, see glm_grouped_stream_decode) in five kernels:
 //
 //   1. route_logits_kernel    router logits (one block per expert, 4 waves
 //                             split d) -- and, in extra blocks, the bf16

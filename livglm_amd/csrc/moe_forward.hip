@@ -555,10 +555,9 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
     }
     return glm_combine_launch(stream, w.y, w.inv, wts, shared_ready, T, top_k, d, out);
   }
-  // general path: dispatch, then the grouped MFMA GEMMs over 128-row tiles
-  // for more than 64 tokens when the shape allows, else the tiled GEMV
-  // kernels over the work list (a few tokens in a 128-row tile would be
-  // mostly padding)
+  // general path: dispatch, then the grouped MFMA GEMMs (streaming or wide)
+  // for more than 64 tokens, and for decode batches that stream_decode takes,
+  // when the shape allows, else the tiled GEMV kernels over the work list
   // (the grouped GEMMs address the FP8 splits of x and h with 32-bit offsets:
   // beyond 4 GiB of split the layer stays on the GEMV kernels)
   const bool grouped = glm_grouped_layer_supported(d, I) && T > 64 && glm_split_fits(T, d) &&

@@ -916,6 +916,17 @@ SMALL_LAYERS = [
     (24, 1536, 16, 4, 1152, 640, (2, 1)),
     (40, 2560, 16, 8, 1280, 1152, (1, 1)),
     (64, 3584, 12, 4, 896, 384, (1, 1)),
+    # the decode kernels from 16 tokens on, where they run: layers of under 32 MB
+    # of reached weights (the larger ones above run on the streaming GEMMs from
+    # 16 tokens) -- the shared tiles in the router's launch, in the expert
+    # kernels, beside the selection; chunk counts 3, 7, 5 / 10
+    (50, 2048, 8, 8, 512, 512, (1, 1)),
+    (16, 2048, 8, 4, 768, 768, (1, 1)),
+    (40, 1024, 32, 8, 512, 512, (1, 1)),
+    (48, 4096, 16, 4, 256, 256, (1, 1)),
+    (32, 1536, 16, 8, 640, 640, (1, 1)),
+    (64, 3584, 4, 4, 896, 384, (1, 1)),
+    (40, 2560, 6, 4, 1280, 1152, (1, 1)),
     # grouped GEMMs whose last gate/up feature tile is half empty, the first one
     # too (I 128), with an odd count of K chunks in the down GEMM
     (65, 512, 8, 2, 128, 0, (1, 1)),
