@@ -68,29 +68,36 @@ struct DenseTile {
 
 // bf16 stages hold 64 of K: token tiles are pairs of blocks a wave there, so
 // that a stage is whole rounds of loads
-template <int FMT>
-constexpr bool dense_takes(int tb) {
-  return FMT != FMT_BF16 || tb % 2 == 0;
+// and MXFP4's need 128 weight rows for that; gate/up tiles hold both projections.
+// 64-row tiles (br 1) are for few tokens.
+template <int FMT, int NPROJ>
+constexpr bool dense_takes(int br, int tb) {
+  return (FMT != FMT_BF16 || tb % 2 == 0) &&
+         (br > 1 || (FMT != FMT_MXFP4 && NPROJ == 1 && tb <= 2));
 }
 
 // The tile that takes the fewest rounds of the CUs, each priced by its size.
 // A workgroup alone on its CU took, in us per 128 of K (MXFP8, K 4096):
 // 0.81 + 0.055 br tb with 256-row tiles (tb 1 / 2 / 3 / 4: 1.04 / 1.23 / 1.46 /
 // 1.68), 0.48 + 0.08 br tb with 128-row ones (0.65 / 0.78 / 0.93 / 1.15); the
-// weights below are these in one unit.  Picked against measured best at
+// weights below are these in one unit.  64-row tiles (tb 1 / 2: 0.43 / 0.52)
+// where those would leave most of the chip idle: 100 tokens at N = K = 4096
+// 15.8 us in MXFP8 and 20.1 in bf16, where 128-row tiles take 20.5 and 26.3.
+// Picked against measured best at
 // N 4096, K 4096: T 1500 (4, 3) 62 us, where (4, 4) takes 70, (2, 3) 68,
 // (4, 2) 93; T 333, N 2048, K 2048: (2, 1) 12 us, (4, 4) 29.
 template <int FMT, int NPROJ>
 static DenseTile dense_tile(int T, int N) {
   DenseTile best{0, 0};
   long long best_cost = 0;
-  for (int br = 4; br >= 2; br -= 2)
+  for (int br = 4; br >= 1; br /= 2)
     for (int tb = 4; tb >= 1; --tb) {
-      if (!dense_takes<FMT>(tb)) continue;
+      if (!dense_takes<FMT, NPROJ>(br, tb)) continue;
       const int feat = 64 * br / NPROJ;
       const long long items = (long long)((N + feat - 1) / feat) * ((T + 32 * tb - 1) / (32 * tb));
       const long long rounds = (items + kDenseCUs - 1) / kDenseCUs;
-      const long long cost = rounds * (br == 4 ? 30 + 2 * br * tb : 18 + 3 * br * tb);
+      const long long cost =
+          rounds * (br == 4 ? 30 + 2 * br * tb : br == 2 ? 18 + 3 * br * tb : 14 + 4 * tb);
       if (!best.br || cost < best_cost) {
         best = DenseTile{br, tb};
         best_cost = cost;
@@ -101,7 +108,7 @@ static DenseTile dense_tile(int T, int N) {
 
 template <int FMT, int NPROJ, int BR, int TB = 4>
 static void launch_dense_rows(hipStream_t stream, const DenseArgs &a, int tb) {
-  if constexpr (dense_takes<FMT>(TB)) {
+  if constexpr (dense_takes<FMT, NPROJ>(BR, TB)) {
     if (tb == TB) return launch_dense_tile<FMT, NPROJ, BR, TB>(stream, a);
   }
   if constexpr (TB > 1) launch_dense_rows<FMT, NPROJ, BR, TB - 1>(stream, a, tb);
@@ -112,8 +119,10 @@ static int launch_dense(hipStream_t stream, const DenseArgs &a) {
   const DenseTile tile = dense_tile<FMT, NPROJ>(a.T, a.N);
   if (tile.br == 4)
     launch_dense_rows<FMT, NPROJ, 4>(stream, a, tile.tb);
-  else
+  else if (tile.br == 2)
     launch_dense_rows<FMT, NPROJ, 2>(stream, a, tile.tb);
+  else
+    launch_dense_rows<FMT, NPROJ, 1>(stream, a, tile.tb);
   GLM_LAUNCH_CHECK("dense_gemm_kernel");
   return GLM_OK;
 }

@@ -66,7 +66,8 @@ struct DenseRaw<FMT_BF16> {
 
 // One stage of the ring: [16 TB WT tokens][kChunk bf16], then
 // [64 BR weight rows][kRow], then (MX) [64 BR] dwords of E8M0 bytes.  WT waves
-// along the tokens; as many stages (2 to 4) as fit KB.
+// along the tokens; as many stages (2 to 8) as fit KB: a small tile's chunk
+// takes the memory latency over the chunks in flight.
 template <int FMT, int BR, int TB, int WT, int KB>
 struct DenseLds {
   using Raw = DenseRaw<FMT>;
@@ -81,11 +82,23 @@ struct DenseLds {
   static constexpr int kXLoads = kX / (1024 * kWaves), kWLoads = kW / (1024 * kWaves);
   static constexpr int kLoads = kXLoads + kWLoads;
   static_assert(kX % (1024 * kWaves) == 0 && kW % (1024 * kWaves) == 0, "staging");
-  static constexpr int kStages = 4 * kStage <= KB * 1024 ? 4 : 3 * kStage <= KB * 1024 ? 3 : 2;
+  static constexpr int kStages = KB * 1024 / kStage < 8 ? KB * 1024 / kStage : 8;
   static constexpr int kBytes = kStages * kStage;
-  static_assert(kBytes <= KB * 1024, "LDS ring exceeds its share");
+  static_assert(kStages >= 2, "LDS ring exceeds its share");
   __device__ static int xswz(int row) { return row & (kXPieces - 1); }
 };
+
+// Waits until at most `ahead` (0 .. MAX, uniform) chunks of LOADS loads are
+// outstanding.
+template <int MAX, int LOADS>
+__device__ __forceinline__ void wait_chunks_ahead(int ahead) {
+  static_assert(MAX * LOADS < 64, "the wait counter's range");
+  if (ahead >= MAX) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(MAX * LOADS));
+  } else if constexpr (MAX > 0) {
+    wait_chunks_ahead<MAX - 1, LOADS>(ahead);
+  }
+}
 
 // One workgroup's work item; lin is its workgroup's index among the launch's
 // dense ones, congruent to blockIdx.x modulo the XCDs.
@@ -198,13 +211,7 @@ __device__ __forceinline__ void dense_item(const DenseArgs &a, int lin) {
   int stage = 0;
   for (int c = 0; c < nchunks; ++c) {
     // (waves that load scales too have more in flight and wait for a little more)
-    const int ahead = min(kS - 2, nchunks - 1 - c);
-    if (kS > 3 && ahead >= 2)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * L::kLoads));
-    else if (kS > 2 && ahead >= 1)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(L::kLoads));
-    else
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    wait_chunks_ahead<kS - 2, L::kLoads>(min(kS - 2, nchunks - 1 - c));
     ring_barrier();
     if (c + kS - 1 < nchunks) issue(c + kS - 1, stage == 0 ? kS - 1 : stage - 1);
     compute(stage);

@@ -875,13 +875,14 @@ int glm_dense_gemm_launch(hipStream_t stream, int nproj, const uint16_t *x, int 
 
 // Whether a resident linear (nproj 1) or the two gate/up projections run as a
 // tiled GEMM (dense_gemm.hip) instead of streaming tiles: from 65 tokens on
-// (MXFP8, K = N = 4096: 20.6 against 21 us at 64 tokens, 25 against 20 at 65,
-// 63 against 21 at 200; the streaming tiles go over the weights once per 64
-// tokens), and at any count where K has no split for the streaming tiles,
+// (K = N = 4096: MXFP4 19.2 against 18.7 us at 64 tokens, MXFP8 63 against 21 at
+// 200; the streaming tiles go over the weights once per 64 tokens), a linear in
+// MXFP8 from 49 on (64 tokens: 15.7 against 20.5 us, at N = K = 2048 9.0 against
+// 10.7; 32 tokens: 15.6 against 13.3), and at any count where K has no split for the streaming tiles,
 // which would leave the scalar kernel.
 static bool dense_gemm_rule(int T, int fmt, int nproj, int K, int N, const uint8_t *s0,
                             const uint8_t *s1) {
-  constexpr int kMinT = 65;
+  const int kMinT = fmt == GLM_FMT_MXFP8 && nproj == 1 ? 49 : 65;
   int ksplit, cpw;
   return (T >= kMinT || !choose_split(fmt, nproj, K, &ksplit, &cpw)) &&
          glm_dense_gemm_supported(T, K, N, fmt, s0, s1);

@@ -47,6 +47,8 @@ def _check(got, want):
     (129, 304, 896), (300, 2064, 128), (520, 1040, 1152),
     # tiles of 256 rows x 96 and 128 tokens: grids near one workgroup per CU
     (1500, 4096, 256), (2100, 4000, 384),
+    # 64-row weight tiles of 32 and 64 tokens (MXFP8 from 49 tokens on, bf16)
+    (49, 1040, 256), (64, 80, 1152), (100, 2048, 512), (128, 4064, 128), (190, 3984, 256),
     # no K split for the streaming tiles: few tokens come here too
     (5, 256, 640), (16, 80, 3328),
 ])
