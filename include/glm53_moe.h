@@ -341,6 +341,22 @@ int glm_limited_swiglu(void *stream, const uint16_t *gate, const uint16_t *up, i
 size_t glm_moe_workspace_bytes(int T, int d, int E, int top_k, int I, int I_shared);
 
 /*
+ * The kernels that glm_moe_forward runs a layer of these sizes on, decided on
+ * the host from the sizes and the alignment of the routed scales (addresses only,
+ * never read): GLM_PATH_*, or a negative status for sizes the layer refuses.
+ * I_shared: the shared expert's width, 0 without one or with shared_in.
+ */
+#define GLM_PATH_FEW_TOKENS 0   /* token-major kernels (T <= 4) */
+#define GLM_PATH_DECODE 1       /* decode kernels (T <= 64) */
+#define GLM_PATH_STREAM_BF16 2  /* streaming grouped GEMMs, bf16 activations */
+#define GLM_PATH_STREAM_SPLIT 3 /* streaming grouped GEMMs, FP8 hi/lo split */
+#define GLM_PATH_WIDE 4         /* wide grouped GEMMs, FP8 hi/lo split */
+#define GLM_PATH_WORK_LIST 5    /* GEMV tiles over the work list */
+int glm_moe_forward_path(int T, int d, int E, int top_k, int I, int I_shared, int shared_fmt,
+                         const uint8_t *gate_scales, const uint8_t *up_scales,
+                         const uint8_t *down_scales);
+
+/*
  * Zero-fills a workspace with a plain kernel (no memset node, so it may be
  * captured in a graph).  glm_moe_forward does not need it; it is provided so
  * callers can give a workspace a defined initial state.  Calls that overlap

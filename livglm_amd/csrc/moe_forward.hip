@@ -287,6 +287,44 @@ extern "C" int glm_moe_workspace_init(void *stream, void *workspace, size_t work
 
 int glm_hc_post_launch(hipStream_t stream, const glm::HcFuse &f, const float *y, int T, int d);
 
+// Which kernels run a layer of these sizes (GLM_PATH_*).  Is: the width of a
+// shared expert that the layer computes itself, 0 for none.  dword_scales: the
+// routed scales lie on 4-byte boundaries; the grouped GEMMs stage them in LDS
+// four at a time, so scales that do not stay on the kernels that read them with
+// ordinary loads.
+static int layer_path(int T, int d, int E, int k, int I, int Is, int shared_fmt,
+                      bool dword_scales) {
+  const int fused_Is = shared_fmt == GLM_FMT_BF16 ? Is : 0;  // an MX one runs by itself
+  if (glm_pair_path_supported(T, d, E, k, I, fused_Is)) return GLM_PATH_FEW_TOKENS;
+  if (dword_scales && glm_grouped_stream_decode(T, d, E, k, I, Is, shared_fmt))
+    return GLM_PATH_STREAM_BF16;
+  if (glm_decode_path_supported(T, d, E, k, I, fused_Is)) return GLM_PATH_DECODE;
+  // the grouped GEMMs address the FP8 splits of x and h with 32-bit offsets:
+  // beyond 4 GiB of split the layer stays on the GEMV kernels
+  const long long P = (long long)T * k;
+  if (!dword_scales || !glm_grouped_layer_supported(d, I) || T <= 64 || !glm_split_fits(T, d) ||
+      !glm_split_fits(P, I))
+    return GLM_PATH_WORK_LIST;
+  if (glm_grouped_layer_tile_rows(P, E, I) == glm_grouped_tile_rows()) return GLM_PATH_WIDE;
+  return glm_grouped_stream_bf16(P, E) ? GLM_PATH_STREAM_BF16 : GLM_PATH_STREAM_SPLIT;
+}
+
+static bool dword_aligned(const uint8_t *a, const uint8_t *b, const uint8_t *c) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 3u) == 0;
+}
+
+extern "C" int glm_moe_forward_path(int T, int d, int E, int top_k, int I, int I_shared,
+                                    int shared_fmt, const uint8_t *gate_scales,
+                                    const uint8_t *up_scales, const uint8_t *down_scales) {
+  glm::clear_error();
+  GLM_REQUIRE(T > 0 && d > 0 && E > 0 && E <= 448 && top_k > 0 && top_k <= E && I > 0 &&
+                  I_shared >= 0 && d % 32 == 0 && I % 32 == 0 && I_shared % 32 == 0,
+              GLM_ERR_INVALID_ARGUMENT, "moe_forward_path: invalid sizes T=%d d=%d E=%d k=%d I=%d",
+              T, d, E, top_k, I);
+  return layer_path(T, d, E, top_k, I, I_shared, shared_fmt,
+                    dword_aligned(gate_scales, up_scales, down_scales));
+}
+
 static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
                             const float *router_weight, const float *router_bias, int E,
                             int top_k, int n_group, int topk_group, int norm_topk_prob,
@@ -498,7 +536,9 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
               "T <= 4, top_k <= 8, d / 512 in {2, 4, 6, 8} and I / 128 in {1, 2, 4, 6, 8, 16} "
               "(T=%d d=%d k=%d I=%d)",
               T, d, top_k, I);
-  if (glm_pair_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0)) {
+  const int path = layer_path(T, d, E, top_k, I, has_shared && !shared_in ? Is : 0, shared_fmt,
+                              dword_aligned(gate_scales, up_scales, down_scales));
+  if (path == GLM_PATH_FEW_TOKENS) {
     // a few tokens: three token-major kernels, no dispatch
     if (has_shared && !shared_in && !shared_bf16) {
       rc = glm_mlp_launch(stream, x, T, d, I_shared, shared_fmt, shared_gate, shared_gate_scales,
@@ -518,9 +558,7 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
     *hc_done = hc != nullptr;  // fused into the down + combine kernel
     return rc;
   }
-  const bool stream_decode = glm_grouped_stream_decode(
-      T, d, E, top_k, I, has_shared && !shared_in ? Is : 0, shared_fmt);
-  if (!stream_decode && glm_decode_path_supported(T, d, E, top_k, I, fuse_shared ? Is : 0)) {
+  if (path == GLM_PATH_DECODE) {
     // decode: six short kernels, no host synchronisation; the bf16 shared
     // expert rides in the two routing kernels, or from 16 tokens on (router
     // logits on MFMA) in the two routed expert kernels
@@ -555,23 +593,15 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
     }
     return glm_combine_launch(stream, w.y, w.inv, wts, shared_ready, T, top_k, d, out);
   }
-  // general path: dispatch, then the grouped MFMA GEMMs (streaming or wide)
-  // for more than 64 tokens, and for decode batches that stream_decode takes,
-  // when the shape allows, else the tiled GEMV kernels over the work list
-  // (the grouped GEMMs address the FP8 splits of x and h with 32-bit offsets:
-  // beyond 4 GiB of split the layer stays on the GEMV kernels)
-  const bool grouped = glm_grouped_layer_supported(d, I) && T > 64 && glm_split_fits(T, d) &&
-                       glm_split_fits((long long)T * top_k, I);
+  // general path: dispatch, then the grouped MFMA GEMMs (streaming or wide), else
+  // the tiled GEMV kernels over the work list
   const long long P = (long long)T * top_k;
-  const int tile_rows = grouped         ? glm_grouped_layer_tile_rows(P, E, I)
-                        : stream_decode ? glm_grouped_stream_rows()
-                                        : 0;
-  const bool wide = tile_rows == glm_grouped_tile_rows();
-  const bool stream_path = stream_decode || (grouped && !wide);
-  const bool stream_bf16 = stream_decode || (stream_path && glm_grouped_stream_bf16(P, E));
+  const bool wide = path == GLM_PATH_WIDE, stream_bf16 = path == GLM_PATH_STREAM_BF16;
+  const bool stream_path = stream_bf16 || path == GLM_PATH_STREAM_SPLIT;
+  const int tile_rows = wide ? glm_grouped_tile_rows() : stream_path ? glm_grouped_stream_rows() : 0;
   // with the bf16 router GEMM, x's FP8 split rides in the router weights'
   // split launch (one kernel, two block ranges)
-  const bool split_x = grouped && !stream_bf16;
+  const bool split_x = wide || path == GLM_PATH_STREAM_SPLIT;
   const bool split_early = split_x && w.router_split != nullptr && glm_router_split_supported(T, d);
   if (split_early) {
     rc = glm_prefill_split_launch(stream, router_weight, E, d, w.router_split, x, T, w.x_split);
@@ -628,7 +658,7 @@ static int moe_forward_core(void *stream_v, const uint16_t *x, int T, int d,
                                           E, down_packed, down_scales, w.y, ride_dn);
     }
     if (ride) shared_ready = w.shared_out;
-  } else if (grouped) {
+  } else if (wide) {
     // a bf16 shared expert on the dense GEMMs: its gate/up tiles ride in the
     // wide routed gate/up launch (after the routed work items)
     shared_fused = has_shared && !shared_in &&

@@ -31,6 +31,13 @@ GLM_ACT_FP6X2 = 1
 GLM_ACT_FP4 = 2
 GLM_ACT_FP8FP6 = 3
 
+GLM_PATH_FEW_TOKENS = 0
+GLM_PATH_DECODE = 1
+GLM_PATH_STREAM_BF16 = 2
+GLM_PATH_STREAM_SPLIT = 3
+GLM_PATH_WIDE = 4
+GLM_PATH_WORK_LIST = 5
+
 GLM_READ_DROP_CACHE = 1
 GLM_HC_BF16_STREAMS = 1
 GLM_NOALLOC_SCRATCH_BYTES = 64 << 20
@@ -73,6 +80,7 @@ SIGNATURES = {
     "glm_mx_dequantize": (_i, [_p, _p, _p, _i, _i, _i, _p]),
     "glm_limited_swiglu": (_i, [_p, _p, _p, _i64, _f, _p]),
     "glm_moe_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i]),
+    "glm_moe_forward_path": (_i, [_i, _i, _i, _i, _i, _i, _i, _p, _p, _p]),
     "glm_moe_workspace_init": (_i, [_p, _p, _sz]),
     "glm_moe_forward": (_i, [_p, _p, _i, _i, _p, _p, _i, _i, _i, _i, _i, _f, _i,
                              _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _p, _p, _p, _p,

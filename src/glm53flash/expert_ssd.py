@@ -179,7 +179,8 @@ class HBMExpertBank:
         """Replaces the whole bank with stacked ``[E, ...]`` checkpoint
         tensors: the packed codes are rewritten in the bank layout
         (``native.mxfp4_tile``), the scales kept as they are (no copy when
-        already contiguous u8 on this device)."""
+        already contiguous u8 on this device and 16-byte aligned, which the
+        kernels ask for: a view into a larger buffer may not be)."""
         self._require_active()
         for name, shape in self.shapes().items():
             src = self._as_bytes(tensors[name])
@@ -191,7 +192,8 @@ class HBMExpertBank:
                 src = src.to(self.device)
             if name.endswith(".weight_packed"):
                 src = N.native.mxfp4_tile(src)
-            self.tensors[name] = src.contiguous()
+            src = src.contiguous()
+            self.tensors[name] = src if src.data_ptr() % 16 == 0 else src.clone()
 
     def projection(self, part: str) -> tuple[torch.Tensor, torch.Tensor]:
         return self.tensors[f"{part}.weight_packed"], self.tensors[f"{part}.weight_scale"]

@@ -76,6 +76,20 @@ def workspace(nbytes: int) -> torch.Tensor:
     return ws
 
 
+PATHS = {getattr(native, n): n[len("GLM_PATH_"):].lower()
+         for n in dir(native) if n.startswith("GLM_PATH_")}
+
+
+def layer_path(shape, T: int | None = None, shared: bool = True,
+               shared_fmt: int = native.GLM_FMT_BF16, scales=(None, None, None)) -> str:
+    """The kernels that glm_moe_forward runs a layer on (a host-side decision):
+    tests that mean one of them assert it."""
+    T = shape.T if T is None else T
+    path = native.load().glm_moe_forward_path(T, shape.d, shape.E, shape.k, shape.I,
+                                              shape.I_shared if shared else 0, shared_fmt, *scales)
+    return PATHS[path]
+
+
 def run_layer(dl: dict[str, torch.Tensor], shape, T: int | None = None, shared: bool = True,
               bias: torch.Tensor | None = None, ws: torch.Tensor | None = None,
               shared_in: torch.Tensor | None = None, shared_fmt: int = native.GLM_FMT_BF16):

@@ -114,6 +114,58 @@ def test_stream_decode_batches(gu, T, d, E, k, I, Is, fmt):
     assert O.rel_l2(gu.host(out)[same], want[same]) < REL_L2
 
 
+@pytest.mark.parametrize("T,d,E,k,I,path,otherwise", [
+    (3, 1024, 16, 2, 512, "few_tokens", "few_tokens"),
+    (64, 1024, 64, 8, 512, "stream_bf16", "decode"),
+    (100, 1024, 8, 2, 256, "stream_bf16", "work_list"),
+    (100, 512, 8, 8, 256, "stream_split", "work_list"),
+])
+def test_routed_scales_off_a_4_byte_boundary(gu, T, d, E, k, I, path, otherwise):
+    # scales that start off a 4-byte boundary are read by other kernels and give
+    # the same layer
+    shape = MoEShape("scales", T, d, E, k, I, 0)
+    layer = make_layer(shape, 7500 + T + d)
+    want, inter = _oracle(layer, shape, None)
+    dl = gu.upload_layer(layer)
+    names = [key for key in BANK_KEYS if key.endswith("scale")]
+    assert gu.layer_path(shape, scales=[dl[key].data_ptr() for key in names]) == path
+    for i, key in enumerate(names):
+        moved = torch_bytes(gu, dl[key].numel() + 4)[i + 1:][:dl[key].numel()]
+        moved.copy_(dl[key].reshape(-1))
+        dl[key] = moved
+    assert gu.layer_path(shape, scales=[dl[key].data_ptr() for key in names]) == otherwise
+    out, w, idx = gu.run_layer(dl, shape, shared=False)
+    same = np.all(gu.host(idx).astype(np.uint32) == inter["indices"], axis=1)
+    assert same.sum() >= T - 1
+    assert O.rel_l2(gu.host(out)[same], want[same]) < REL_L2
+
+
+def torch_bytes(gu, n):
+    return gu.to_dev(np.zeros(n, dtype=np.uint8))
+
+
+def test_bank_keeps_scales_on_aligned_memory(gu):
+    # load_bank takes a view that starts off the kernels' alignment by copying it
+    from glm53flash.expert_ssd import HBMExpertBank
+    shape = MoEShape("bank", 1, 512, 4, 2, 128, 0)
+    layer = make_layer(shape, 7600)
+    bank = HBMExpertBank(layer=0, num_experts=4, hidden_size=512, intermediate_size=128,
+                         swiglu_limit=10.0, device="cuda")
+    tensors = {key: gu.to_dev(layer[key]) for key in BANK_KEYS}
+    kept = {}
+    for key in BANK_KEYS:
+        if key.endswith("scale"):
+            n = tensors[key].numel()
+            kept[key] = tensors[key]
+            tensors[key] = torch_bytes(gu, n + 1)[1:].copy_(kept[key].reshape(-1)).reshape(kept[key].shape)
+    bank.load_bank(tensors)
+    for key, scales in kept.items():
+        assert bank.tensors[key].data_ptr() % 16 == 0
+        assert np.array_equal(gu.host(bank.tensors[key]), gu.host(scales))
+    bank.load_bank({**tensors, **kept})  # aligned scales are not copied
+    assert all(bank.tensors[key].data_ptr() == kept[key].data_ptr() for key in kept)
+
+
 def test_stream_gemms_equal_the_wide_forms(gu):
     """Bit for bit: the layer's routed output against the wide grouped GEMMs
     called by themselves on the same split, tiles and weights."""

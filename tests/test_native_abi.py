@@ -286,6 +286,29 @@ def test_entry_points_of_even_chunk_counts_refuse_others(lib, d, I, Is):
                 1, 1, 1, 2.5, fake, d, I, fake, fake, fake, fake, 10.0, fake, fake, fake)
 
 
+@pytest.mark.parametrize("T,aligned,otherwise", [
+    (2, "FEW_TOKENS", "FEW_TOKENS"), (64, "STREAM_BF16", "DECODE"),
+    (333, "STREAM_BF16", "WORK_LIST"), (1200, "STREAM_SPLIT", "WORK_LIST"),
+    (4096, "WIDE", "WORK_LIST")])
+def test_routed_scales_off_a_4_byte_boundary_leave_the_grouped_gemms(lib, T, aligned, otherwise):
+    # the grouped GEMMs stage four scales at a time straight into LDS; the other
+    # kernels read them with ordinary loads
+    def path(*offsets):
+        return lib.glm_moe_forward_path(T, 2048, 128, 8, 768, 768, native.GLM_FMT_BF16,
+                                        *(0x1000 + o for o in offsets))
+
+    assert path(0, 0, 0) == path(4, 8, 12) == getattr(native, "GLM_PATH_" + aligned)
+    for offsets in ((1, 0, 0), (0, 2, 0), (0, 0, 3)):
+        assert path(*offsets) == getattr(native, "GLM_PATH_" + otherwise)
+
+
+def test_forward_path_refuses_what_the_layer_refuses(lib):
+    for sizes in ((0, 2048, 128, 8, 768, 0), (2, 2040, 128, 8, 768, 0), (2, 2048, 449, 8, 768, 0),
+                  (2, 2048, 4, 8, 768, 0), (2, 2048, 128, 8, 768, 40)):
+        _expect(native.GLM_ERR_INVALID_ARGUMENT, "glm_moe_forward_path", *sizes,
+                native.GLM_FMT_BF16, None, None, None)
+
+
 def test_split_beyond_32_bit_offsets_is_rejected_on_host(lib):
     # the grouped GEMMs address an activation split through 32-bit offsets: a
     # split above 4 GiB is refused instead of read as zeros past the limit
