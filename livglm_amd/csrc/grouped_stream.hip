@@ -30,6 +30,7 @@
 // split form) 123 us where its two products as launches of their own made it
 // 152, at 1500 (E 120, d 1536) 138 and 163.
 #include <algorithm>
+#include <cmath>
 
 #include "act_split.h"
 #include "dense_tile.h"
@@ -542,16 +543,47 @@ int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, l
 }
 
 // Whether the decode layer (16 to 64 tokens, the router's logits on MFMA) runs
-// on the streaming form instead of the decode kernels, which go over K in one
-// round of loads a workgroup and run an MX shared expert by itself.  At d 4096,
-// E 288, k 8, I 2048: 16 / 24 / 32 / 64 tokens 298 / 383 / 432 / 573 us (decode
-// kernels 301 / 409 / 498 / 723); d 2048, E 128, I 768: 63.9 / 74.6 / 76.1 / 86.9
-// (64.3 / 75.3 / 79.8 / 91.5), with an MXFP8 shared expert 63.6 / 74.5 / 75.9 /
-// 86.5 (74.2 / 87.4 / 93.9 / 110.8).  A layer of a few MB is launches either way
-// (d 1024, E 16, I 512: 33.3 and 32.8) and stays but for the MX shared expert's
-// own launches (33.2 and 39.0).
-bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt) {
+// on the streaming form instead of the decode kernels (decode_kernels: they take
+// the layer), which go over K in one round of loads a workgroup and run an MX
+// shared expert by itself.  At d 4096, E 288, k 8, I 2048: 16 / 24 / 32 / 64 tokens
+// 298 / 383 / 432 / 573 us (decode kernels 301 / 409 / 498 / 723); d 2048, E 128,
+// I 768: 63.9 / 74.6 / 76.1 / 86.9 (64.3 / 75.3 / 79.8 / 91.5), with an MXFP8 shared
+// expert 63.6 / 74.5 / 75.9 / 86.5 (74.2 / 87.4 / 93.9 / 110.8).
+//
+// A streaming workgroup takes 128 features over all of K, a decode workgroup 16
+// over a quarter of it, so the streaming form needs work items for the CUs.
+// Counted for uniform routing, which 16 or more tokens come close to: items of
+// the gate/up launch and rows per expert reached.  Layer times, decode kernels
+// against streaming form, bf16 shared expert / none (d, E, k, I: tokens, items, rows):
+//   4096, 16, 4, 512:  48, 64, 12    52 : 65 us /  46 : 52
+//   2048, 32, 4, 512:  48, 128, 6    36 : 43    /  34 : 34
+//   2048, 24, 8, 768:  32, 144, 11   43 : 44    /  39 : 36;  64, 144, 21  55 : 47 / 49 : 39
+//   1024, 64, 4, 512:  16, 165, 1.6  28 : 30    /  27 : 28;  64, 252, 4   35 : 36 / 31 : 28
+//   4096, 48, 8, 512:  48, 192, 8    77 : 73    /  71 : 60
+//   4096, 64, 4, 512:  32, 224, 2.3              71 : 63;  64, 252, 4   82 : 90
+//   3072, 64, 6, 512:  32, 245, 3    61 : 71    /  57 : 53
+//   4096, 32, 8, 1024: 16, 253, 4    80 : 90    /  77 : 63;  64, 256, 16 129 : 94 / 109 : 69
+// a little more than an item per CU makes some take two:
+//   2048, 64, 2, 1024: 32, 327, 1.6  50 : 56    /  49 : 53
+//   4096, 24, 8, 2048: 22, 384, 7   130 : 98
+// and from 400 items on the streaming form is level or better throughout.  Below
+// 32 MB of weights the layer is launches either way (d 1024, E 16, k 2, I 512, 32
+// tokens: 23 : 30 / 21 : 25).  An MX shared expert costs the decode kernels two
+// launches more, which only few, long items outweigh (MXFP8; 4096, 16, 4, 512: 16
+// tokens 54 : 58 us, 20 58 : 59, 32 61 : 60; 1024, 16, 2, 512, 16 tokens 29 : 28).
+bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt,
+                               bool decode_kernels) {
   if (T < 16 || T > kStreamRows || d % 512 != 0 || I % 128 != 0) return false;
-  const double weights = 1.5 * std::min((long long)E, (long long)T * k) * d * I;
-  return weights >= 32e6 || (Is > 0 && shared_fmt != GLM_FMT_BF16);
+  const bool heavy = 1.5 * std::min((long long)E, (long long)T * k) * d * I >= 32e6;
+  const bool mx = Is > 0 && shared_fmt != GLM_FMT_BF16;
+  if (!decode_kernels) return heavy || mx;
+  const double reached = E * (1.0 - std::pow(1.0 - (double)k / E, T));
+  const double items = reached * (I / 128), rows = T * k / reached;
+  if (mx) return T >= 24 || items >= 96 || d <= 1024;
+  if (!heavy) return false;
+  if (items >= 400) return true;
+  if (items > kStreamCUs && rows < 4) return false;
+  // (the shared expert's own items need room beside the routed ones)
+  if (T >= (Is > 0 ? 32 : 24)) return items >= 115 + d / ((Is > 0 ? 7 : 30) * rows);
+  return items >= 180 && items * rows >= (Is > 0 ? 1400 : 1000);
 }

@@ -86,7 +86,8 @@ int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, l
                                         const int4 *tiles, const int32_t *num_tiles, int max_tiles,
                                         int I, int d, int E, const uint8_t *dw, const uint8_t *ds,
                                         uint16_t *y, const glm::RidingGemm *ride);
-bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt);
+bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt,
+                               bool decode_kernels);
 bool glm_dense_gemm_supported(int T, int K, int N, int fmt, const uint8_t *s0, const uint8_t *s1);
 int glm_gate_up_launch(hipStream_t stream, const uint16_t *x, int T, int d, int I, int E, int k,
                        const uint8_t *gw, const uint8_t *gs, const uint8_t *uw, const uint8_t *us,
@@ -296,9 +297,10 @@ static int layer_path(int T, int d, int E, int k, int I, int Is, int shared_fmt,
                       bool dword_scales) {
   const int fused_Is = shared_fmt == GLM_FMT_BF16 ? Is : 0;  // an MX one runs by itself
   if (glm_pair_path_supported(T, d, E, k, I, fused_Is)) return GLM_PATH_FEW_TOKENS;
-  if (dword_scales && glm_grouped_stream_decode(T, d, E, k, I, Is, shared_fmt))
+  const bool decode_kernels = glm_decode_path_supported(T, d, E, k, I, fused_Is);
+  if (dword_scales && glm_grouped_stream_decode(T, d, E, k, I, Is, shared_fmt, decode_kernels))
     return GLM_PATH_STREAM_BF16;
-  if (glm_decode_path_supported(T, d, E, k, I, fused_Is)) return GLM_PATH_DECODE;
+  if (decode_kernels) return GLM_PATH_DECODE;
   // the grouped GEMMs address the FP8 splits of x and h with 32-bit offsets:
   // beyond 4 GiB of split the layer stays on the GEMV kernels
   const long long P = (long long)T * k;

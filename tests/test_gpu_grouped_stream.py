@@ -100,10 +100,14 @@ def test_stream_layer_row_and_chunk_edges(gu, d, I, Is, k, fmt):
     # shared expert, one that cannot ride (I_shared 96)
     (16, 1024, 64, 8, 512, 512, native.GLM_FMT_MXFP8), (64, 2048, 32, 8, 768, 768, native.GLM_FMT_BF16),
     (64, 1024, 8, 8, 1280, 128, native.GLM_FMT_MXFP4), (33, 512, 16, 2, 128, 128, native.GLM_FMT_MXFP8),
-    (17, 2560, 48, 6, 640, 0, None), (40, 2048, 24, 8, 1024, 96, native.GLM_FMT_BF16),
+    (33, 2560, 48, 6, 640, 0, None), (40, 2048, 24, 8, 1024, 96, native.GLM_FMT_BF16),
+    # too few work items: the decode kernels
+    (17, 2560, 48, 6, 640, 0, None),
 ])
 def test_stream_decode_batches(gu, T, d, E, k, I, Is, fmt):
     shape = MoEShape("decode", T, d, E, k, I, Is)
+    assert gu.layer_path(shape, shared=fmt is not None, shared_fmt=fmt or 0) == \
+        ("decode" if T == 17 else "stream_bf16")
     layer = make_layer(shape, 7300 + T + d)
     shared = _shared_weights(layer, fmt)
     want, inter = _oracle(layer, shape, shared)

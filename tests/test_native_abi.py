@@ -302,6 +302,24 @@ def test_routed_scales_off_a_4_byte_boundary_leave_the_grouped_gemms(lib, T, ali
         assert path(*offsets) == getattr(native, "GLM_PATH_" + otherwise)
 
 
+@pytest.mark.parametrize("T,d,E,k,I,bf16,mx", [
+    # T, d, E, k, I, path with a bf16 shared expert and with an MXFP8 one:
+    # few work items for the streaming GEMMs' workgroups
+    (48, 4096, 16, 4, 512, "DECODE", "STREAM_BF16"), (16, 4096, 16, 4, 512, "DECODE", "DECODE"),
+    (64, 2048, 32, 4, 512, "DECODE", "STREAM_BF16"), (40, 2048, 256, 2, 512, "DECODE", "STREAM_BF16"),
+    (32, 2048, 64, 2, 1024, "DECODE", "STREAM_BF16"), (16, 1024, 64, 4, 512, "DECODE", "STREAM_BF16"),
+    # enough of them, or many rows an expert
+    (64, 2048, 24, 8, 768, "STREAM_BF16", "STREAM_BF16"), (64, 4096, 32, 8, 1024, "STREAM_BF16", "STREAM_BF16"),
+    (16, 2048, 128, 8, 768, "STREAM_BF16", "STREAM_BF16"), (16, 4096, 288, 8, 2048, "STREAM_BF16", "STREAM_BF16"),
+    # a layer of a few MB
+    (32, 1024, 16, 2, 512, "DECODE", "STREAM_BF16"), (15, 4096, 288, 8, 2048, "DECODE", "DECODE"),
+])
+def test_decode_batches_stream_where_the_grid_fills(lib, T, d, E, k, I, bf16, mx):
+    for fmt, path in ((native.GLM_FMT_BF16, bf16), (native.GLM_FMT_MXFP8, mx)):
+        assert lib.glm_moe_forward_path(T, d, E, k, I, I, fmt, None, None, None) == \
+            getattr(native, "GLM_PATH_" + path), (path, fmt)
+
+
 def test_forward_path_refuses_what_the_layer_refuses(lib):
     for sizes in ((0, 2048, 128, 8, 768, 0), (2, 2040, 128, 8, 768, 0), (2, 2048, 449, 8, 768, 0),
                   (2, 2048, 4, 8, 768, 0), (2, 2048, 128, 8, 768, 40)):
