@@ -542,6 +542,8 @@ int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, l
   return stream_launch<1, true>(stream, a, max_tiles, E, ride);
 }
 
+bool glm_gemv_splits(int d, int I);
+
 // Whether the decode layer (16 to 64 tokens, the router's logits on MFMA) runs
 // on the streaming form instead of the decode kernels (decode_kernels: they take
 // the layer), which go over K in one round of loads a workgroup and run an MX
@@ -571,12 +573,17 @@ int glm_grouped_stream_down_bf16_launch(hipStream_t stream, const uint16_t *h, l
 // tokens: 23 : 30 / 21 : 25).  An MX shared expert costs the decode kernels two
 // launches more, which only few, long items outweigh (MXFP8; 4096, 16, 4, 512: 16
 // tokens 54 : 58 us, 20 58 : 59, 32 61 : 60; 1024, 16, 2, 512, 16 tokens 29 : 28).
+//
+// Where the decode kernels do not take the layer, the other choice is the GEMV
+// tiles over the work list; the streaming form is taken whatever the size where
+// these have no K split (d 1024, E 8, k 2, I 1408, 32 tokens: 27.5 us, one thread per
+// output 2945).
 bool glm_grouped_stream_decode(int T, int d, int E, int k, int I, int Is, int shared_fmt,
                                bool decode_kernels) {
   if (T < 16 || T > kStreamRows || d % 512 != 0 || I % 128 != 0) return false;
   const bool heavy = 1.5 * std::min((long long)E, (long long)T * k) * d * I >= 32e6;
   const bool mx = Is > 0 && shared_fmt != GLM_FMT_BF16;
-  if (!decode_kernels) return heavy || mx;
+  if (!decode_kernels) return heavy || mx || !glm_gemv_splits(d, I);
   const double reached = E * (1.0 - std::pow(1.0 - (double)k / E, T));
   const double items = reached * (I / 128), rows = T * k / reached;
   if (mx) return T >= 24 || items >= 96 || d <= 1024;

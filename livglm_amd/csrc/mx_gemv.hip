@@ -888,6 +888,14 @@ static bool dense_gemm_rule(int T, int fmt, int nproj, int K, int N, const uint8
          glm_dense_gemm_supported(T, K, N, fmt, s0, s1);
 }
 
+// Whether the GEMV tiles over the work list have a K split for the routed
+// gate/up (K = d) and down (K = I); without one they run one thread per output.
+bool glm_gemv_splits(int d, int I) {
+  int ksplit, cpw;
+  return choose_split(GLM_FMT_MXFP4, 2, d, &ksplit, &cpw) &&
+         choose_split(GLM_FMT_MXFP4, 1, I, &ksplit, &cpw);
+}
+
 int glm_linear_launch(hipStream_t stream, const uint16_t *x, int T, int in_dims,
                       const void *weight, const uint8_t *scales, int fmt, int out_dims,
                       uint16_t *y) {

@@ -101,6 +101,9 @@ def test_stream_layer_row_and_chunk_edges(gu, d, I, Is, k, fmt):
     (16, 1024, 64, 8, 512, 512, native.GLM_FMT_MXFP8), (64, 2048, 32, 8, 768, 768, native.GLM_FMT_BF16),
     (64, 1024, 8, 8, 1280, 128, native.GLM_FMT_MXFP4), (33, 512, 16, 2, 128, 128, native.GLM_FMT_MXFP8),
     (33, 2560, 48, 6, 640, 0, None), (40, 2048, 24, 8, 1024, 96, native.GLM_FMT_BF16),
+    # small layers that neither the decode kernels nor the GEMV tiles split
+    (32, 1024, 8, 2, 1408, 1408, native.GLM_FMT_BF16), (16, 512, 8, 2, 1664, 0, None),
+    (20, 6656, 8, 2, 256, 0, None),
     # too few work items: the decode kernels
     (17, 2560, 48, 6, 640, 0, None),
 ])

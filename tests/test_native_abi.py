@@ -320,6 +320,16 @@ def test_decode_batches_stream_where_the_grid_fills(lib, T, d, E, k, I, bf16, mx
             getattr(native, "GLM_PATH_" + path), (path, fmt)
 
 
+@pytest.mark.parametrize("T,d,I,path", [
+    (32, 1024, 1408, "STREAM_BF16"), (16, 1024, 1664, "STREAM_BF16"), (64, 512, 1792, "STREAM_BF16"),
+    (20, 6656, 256, "STREAM_BF16"), (32, 512, 512, "WORK_LIST"), (15, 1024, 1408, "WORK_LIST")])
+def test_small_layers_without_a_gemv_split_stream(lib, T, d, I, path):
+    # widths that the decode kernels do not take and whose K the GEMV tiles
+    # cannot split (11, 13, 14 and 15 chunks of 128, 52): one thread per output else
+    assert lib.glm_moe_forward_path(T, d, 8, 2, I, 0, native.GLM_FMT_BF16, None, None, None) == \
+        getattr(native, "GLM_PATH_" + path)
+
+
 def test_forward_path_refuses_what_the_layer_refuses(lib):
     for sizes in ((0, 2048, 128, 8, 768, 0), (2, 2040, 128, 8, 768, 0), (2, 2048, 449, 8, 768, 0),
                   (2, 2048, 4, 8, 768, 0), (2, 2048, 128, 8, 768, 40)):
