@@ -386,15 +386,48 @@ int glm_grouped_stream_rows() { return kStreamRows; }
 // against 845 / 918 us; E 128, 44 rows 150 and 149; E 120, 75 rows 141 and 139).
 bool glm_grouped_stream_bf16(long long pairs, int E) { return pairs <= 48LL * E; }
 
-// Rows per tile of the layer's grouped GEMMs: the streaming form's up to 88
-// rows an expert (layer at 75 rows, d 1536, E 120, I 640: 140 against 159 us;
-// at 94, d 2048, E 128, I 768: 216 against 211) and while the wide forms'
-// tiles (256 features by at most glm_grouped_tile_rows rows) are fewer than the
-// CUs (E 16, I 512, 250 rows: 70 against 90 us, 500 rows: 97 against 101).
-int glm_grouped_layer_tile_rows(long long pairs, int E, int I) {
+// How well the wide forms' items fill the CUs: the share of whole rounds of them,
+// with half the weight on how full the tiles' rows are (an item's time is its K
+// loop before it is its rows).  The rows of an expert are taken a tenth above the
+// average, since a tile more on some experts starts a round.
+static double wide_fill(long long pairs, int E, int d, int I) {
+  const int tile_rows = glm_grouped_tile_rows();
+  const double tiles = E * std::ceil(1.1 * pairs / E / tile_rows);
+  const double gate_up = tiles * ((I + 255) / 256), down = tiles * d / 512;
+  auto rounds = [](double items) { return std::ceil(items / kStreamCUs); };
+  const double full = (gate_up * d + down * I) / kStreamCUs / (rounds(gate_up) * d + rounds(down) * I);
+  return full * (0.5 + 0.5 * pairs / (tiles * tile_rows));
+}
+
+// Rows per tile of the layer's grouped GEMMs, the streaming form's or the wide
+// forms' (256 features by at most glm_grouped_tile_rows rows).  Layer times, wide
+// against streaming.
+//
+// Up to 88 rows an expert the streaming form (75 rows, d 1536, E 120, I 640: 159 :
+// 140 us; at 94, d 2048, E 128, I 768: 211 : 216), but not above 60 rows at long K
+// where the wide forms fill at least two rounds (d 4096, E 288, I 2048, MXFP8 shared
+// expert: 58 rows 1395 : 1383 us, 64 rows 1435 : 1570; d 5120, E 128, I 1536: 56 rows
+// 636 : 634, 75 rows 698 : 782; rounds 0.78 full, E 160, I 1280: 70 rows 612 : 605).
+//
+// Above, the streaming form while the wide forms' items are fewer than the CUs and
+// fill them badly (bf16 shared expert; d 1024, E 16, k 2, I 512: 256 rows, fill 0.23, 91 :
+// 70 us, 512 rows, 0.45, 99 : 97, 1024 rows, 0.9, 131 : 152; d 1024, E 8, k 2, I 256: 1024
+// rows, 0.27, 89 : 78, 4096 rows, 0.85, 165 : 189; d 2048, E 24, k 8, I 768: 333 rows, 0.61,
+// 150 : 130; d 2048, E 64, k 8, I 512: 175 rows, 0.77, 155 : 135; d 4096, where K is
+// longer: E 16, k 4, I 1024: 350 rows, 0.65, 258 : 247, 500 rows, 0.89, 310 : 334; E 8, k 2,
+// I 2048: 400 rows, 0.69, 289 : 317).
+int glm_grouped_layer_tile_rows(long long pairs, int E, int d, int I) {
   const int wide = glm_grouped_tile_rows();
-  const long long wide_items = std::max((long long)E, pairs / wide) * ((I + 255) / 256);
-  return pairs <= 88LL * E || wide_items < kStreamCUs ? kStreamRows : wide;
+  const int features = (I + 255) / 256;
+  const bool long_k = d >= 4096;
+  bool stream;
+  if (pairs <= 88LL * E)
+    stream = !(long_k && pairs > 60LL * E && E * features >= 2 * kStreamCUs &&
+               wide_fill(pairs, E, d, I) >= 0.65);
+  else
+    stream = std::max((long long)E, pairs / wide) * features < kStreamCUs &&
+             wide_fill(pairs, E, d, I) < (long_k ? 0.68 : 0.8);
+  return stream ? kStreamRows : wide;
 }
 
 template <int NPROJ, bool BF, int FMT>

@@ -49,7 +49,7 @@ int glm_dispatch_launch(hipStream_t stream, const uint32_t *indices, int T, int 
                         int32_t *chunk_scratch);
 size_t glm_dispatch_chunk_ints(long long P, int E);
 int glm_grouped_tile_rows();
-int glm_grouped_layer_tile_rows(long long pairs, int E, int I);
+int glm_grouped_layer_tile_rows(long long pairs, int E, int d, int I);
 int glm_grouped_stream_rows();
 bool glm_grouped_stream_bf16(long long pairs, int E);
 bool glm_grouped_layer_supported(int d, int I);
@@ -307,7 +307,7 @@ static int layer_path(int T, int d, int E, int k, int I, int Is, int shared_fmt,
   if (!dword_scales || !glm_grouped_layer_supported(d, I) || T <= 64 || !glm_split_fits(T, d) ||
       !glm_split_fits(P, I))
     return GLM_PATH_WORK_LIST;
-  if (glm_grouped_layer_tile_rows(P, E, I) == glm_grouped_tile_rows()) return GLM_PATH_WIDE;
+  if (glm_grouped_layer_tile_rows(P, E, d, I) == glm_grouped_tile_rows()) return GLM_PATH_WIDE;
   return glm_grouped_stream_bf16(P, E) ? GLM_PATH_STREAM_BF16 : GLM_PATH_STREAM_SPLIT;
 }
 

@@ -320,6 +320,24 @@ def test_decode_batches_stream_where_the_grid_fills(lib, T, d, E, k, I, bf16, mx
             getattr(native, "GLM_PATH_" + path), (path, fmt)
 
 
+@pytest.mark.parametrize("T,d,E,k,I,path", [
+    # hundreds of rows an expert: wide where its items fill the CUs
+    (2048, 1024, 16, 2, 512, "STREAM_SPLIT"), (8192, 1024, 16, 2, 512, "WIDE"),
+    (4096, 1024, 8, 2, 256, "STREAM_SPLIT"), (16384, 1024, 8, 2, 256, "WIDE"),
+    (700, 4096, 16, 4, 1024, "STREAM_SPLIT"), (2000, 4096, 16, 4, 1024, "WIDE"),
+    (1600, 4096, 8, 2, 2048, "WIDE"), (1000, 2048, 24, 8, 768, "STREAM_SPLIT"),
+    (1400, 2048, 64, 8, 512, "STREAM_SPLIT"), (2048, 2048, 64, 8, 512, "WIDE"),
+    # fewer rows: the streaming form, but at long K over full rounds
+    (2100, 4096, 288, 8, 2048, "STREAM_SPLIT"), (2300, 4096, 288, 8, 2048, "WIDE"),
+    (1200, 5120, 128, 8, 1536, "WIDE"), (1400, 4096, 160, 8, 1280, "STREAM_SPLIT"),
+    (1023, 4096, 288, 8, 2048, "STREAM_BF16"), (1400, 2048, 128, 8, 768, "STREAM_SPLIT"),
+    (1500, 2048, 128, 8, 768, "WIDE"),
+])
+def test_layers_run_wide_where_its_items_fill_the_chip(lib, T, d, E, k, I, path):
+    assert lib.glm_moe_forward_path(T, d, E, k, I, I, native.GLM_FMT_BF16, None, None, None) == \
+        getattr(native, "GLM_PATH_" + path)
+
+
 @pytest.mark.parametrize("T,d,I,path", [
     (32, 1024, 1408, "STREAM_BF16"), (16, 1024, 1664, "STREAM_BF16"), (64, 512, 1792, "STREAM_BF16"),
     (20, 6656, 256, "STREAM_BF16"), (32, 512, 512, "WORK_LIST"), (15, 1024, 1408, "WORK_LIST")])
