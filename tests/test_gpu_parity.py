@@ -464,17 +464,20 @@ def test_grouped_expert_gemms_parity(gu):
     assert O.rel_l2(y_got, y_want) < REL_L2 and np.mean(y_got == y_want) > 0.97
 
 
-def test_moe_forward_grouped_equals_public_composition(gu):
-    # glm_moe_forward's grouped path (multi-workgroup dispatch, h split fused
+@pytest.mark.parametrize("T,d,E,k,path", [(400, 1024, 32, 4, "stream_split"),
+                                          (2850, 512, 256, 8, "wide")])
+def test_moe_forward_grouped_equals_public_composition(gu, T, d, E, k, path):
+    # glm_moe_forward's grouped path (either form) (multi-workgroup dispatch, h split fused
     # into the gate/up epilogue) must equal, bit for bit, the public entry
     # points composed by hand on the forward's own route: dispatch, tiles, x
     # split, gate/up to bf16 h, split of h, down, combine.  Its route (bf16
     # MFMA on the f32 router weights split three ways) is checked against the
     # oracle's.
     torch = _torch()
-    shape = MoEShape("grouped", 400, 1024, 32, 4, 256, 0)
+    shape = MoEShape("grouped", T, d, E, k, 256, 0)
+    assert gu.layer_path(shape, shared=False) == path
     layer = make_layer(shape, 1718)
-    T, k, E, d, I = shape.T, shape.k, shape.E, shape.d, shape.I
+    I = shape.I
     P = T * k
     dl = gu.upload_layer(layer)
     lib = native.load()
@@ -676,7 +679,7 @@ def test_moe_layer_nan_gate_scale(gu, T, d, E, k, I, Is):
     # one routed expert's gate row with a NaN scale byte (E8M0 255): its gate
     # value is NaN beside a finite up value, the NaN passes the SwiGLU clamp and
     # every output of the tokens routed to that expert is NaN -- on the
-    # few-token, decode and grouped paths, as in the oracle
+    # few-token path and the streaming one, as in the oracle
     shape = MoEShape("nan_scale", T, d, E, k, I, Is)
     layer = make_layer(shape, 6100 + T)
     _, _, i0, _ = O.router(O.bf16_bits_to_f32(layer["x"]), layer["router_weight"],
@@ -871,19 +874,18 @@ SMALL_LAYERS = [
     (4, 2048, 448, 8, 128, 256, (1, 1)),
     (5, 1024, 64, 6, 256, 256, (1, 1)),
     (9, 2048, 96, 5, 384, 0, (3, 2)),
-    # grouped MFMA GEMMs (T > 64): partial tiles, experts spanning two tiles
+    # streaming grouped GEMMs (T > 64): partial tiles, experts spanning two tiles
     (96, 1024, 16, 4, 256, 256, (1, 1)),
     (600, 1024, 16, 4, 256, 256, (1, 1)),
     (200, 2048, 64, 8, 768, 0, (4, 2)),
     # many pairs: the multi-workgroup dispatch (6 chunks of 1024 pairs, the last partial)
     (700, 1024, 32, 8, 256, 0, (1, 1)),
-    # the decode path beyond 16 tokens (MFMA router, per-token selection, token groups)
+    # decode batches on the streaming grouped GEMMs
     (40, 1024, 64, 8, 512, 512, (1, 1)),
-    # 33-64 tokens at d % 2048 == 0: the shared gate/up tiles in the router's
-    # launch (a partial last token tile and token group)
     (50, 2048, 64, 8, 768, 768, (1, 1)),
-    # 16-32 tokens: the shared expert's tiles in the routed expert kernels (two
-    # chunks per shared down K range; one chunk at I_shared 128, two token groups)
+    # 16-32 tokens on the decode kernels: the shared expert's tiles in the routed
+    # expert kernels (two chunks per shared down K range; one chunk at I_shared
+    # 128, two token groups)
     (16, 2048, 64, 8, 768, 768, (1, 1)),
     (24, 1024, 32, 4, 256, 128, (2, 1)),
     (32, 4096, 24, 8, 2048, 1024, (1, 1)),
@@ -901,7 +903,7 @@ SMALL_LAYERS = [
     (65, 1536, 16, 8, 256, 256, (1, 1)),
     # the real GLM expert geometry (d 4096, I 2048: 16 chunks of 128 in the down
     # projection): E 288 on the few-token path; 64 tokens over 24 experts on the
-    # decode path (~21 pairs per expert, two 16-row h batches)
+    # streaming form (~21 pairs per expert)
     (2, 4096, 288, 8, 2048, 2048, (1, 1)),
     (64, 4096, 24, 8, 2048, 2048, (1, 1)),
     # every chunk count of the few-token and the decode kernels that is not a
@@ -916,9 +918,9 @@ SMALL_LAYERS = [
     (24, 1536, 16, 4, 1152, 640, (2, 1)),
     (40, 2560, 16, 8, 1280, 1152, (1, 1)),
     (64, 3584, 12, 4, 896, 384, (1, 1)),
-    # the decode kernels from 16 tokens on, where they run: layers of under 32 MB
-    # of reached weights (the larger ones above run on the streaming GEMMs from
-    # 16 tokens) -- the shared tiles in the router's launch, in the expert
+    # the decode kernels from 16 tokens on, where they run: layers of few work
+    # items or under 32 MB of reached weights (the others above run on the
+    # streaming GEMMs from 16 tokens) -- the shared tiles in the router's launch, in the expert
     # kernels, beside the selection; chunk counts 3, 7, 5 / 10
     (50, 2048, 8, 8, 512, 512, (1, 1)),
     (16, 2048, 8, 4, 768, 768, (1, 1)),
@@ -927,8 +929,7 @@ SMALL_LAYERS = [
     (32, 1536, 16, 8, 640, 640, (1, 1)),
     (64, 3584, 4, 4, 896, 384, (1, 1)),
     (40, 2560, 6, 4, 1280, 1152, (1, 1)),
-    # grouped GEMMs whose last gate/up feature tile is half empty, the first one
-    # too (I 128), with an odd count of K chunks in the down GEMM
+    # streaming grouped GEMMs over an odd count of K chunks in the down GEMM
     (65, 512, 8, 2, 128, 0, (1, 1)),
     (100, 1536, 8, 4, 384, 384, (1, 1)),
     (300, 1024, 8, 4, 640, 640, (1, 1)),
@@ -963,9 +964,10 @@ def test_moe_layer_small_shapes(gu, T, d, E, k, I, Is, groups):
 
 
 def test_moe_layer_grouped_skewed_routing(gu):
-    # Zipf-biased routing: a few experts take several 128-row tiles, many take
-    # one partial tile or none
+    # Zipf-biased routing: a few experts take several row tiles of the streaming
+    # GEMMs, many take one partial tile or none
     shape = MoEShape("skew", 512, 1024, 32, 4, 256, 256, routing="zipf")
+    assert gu.layer_path(shape) == "stream_split"
     layer = make_layer(shape, 4711)
     want, inter = _oracle_layer(layer, shape)
     counts = np.bincount(inter["indices"].reshape(-1).astype(np.int64), minlength=shape.E)
@@ -1015,6 +1017,7 @@ def test_moe_layer_golden_vectors(gu):
 
 def test_moe_layer_prefill_sampled(gu):
     shape = SHAPES["prefill_t4096"]
+    assert gu.layer_path(shape) == "wide"
     layer = make_layer(shape, 5303)
     out, w, idx = gu.run_layer(gu.upload_layer(layer), shape)
     x = O.bf16_bits_to_f32(layer["x"])

@@ -60,19 +60,24 @@ def _both(shape, seed):
     return res
 
 
-# pairs of calls in a row, the second smaller: the decode path (64 tokens)
-# then the few-token path (2 tokens); the grouped GEMM path (300 tokens) then
-# 96 tokens on the same kernels
+# pairs of calls in a row, the second smaller: a decode batch (64 tokens, the
+# streaming GEMMs on bf16 activations) then the few-token path (2 tokens); the
+# streaming GEMMs on the split (300 tokens) then 96 tokens on bf16; the wide
+# GEMMs (720 tokens) then the decode kernels (24 tokens)
 SEQUENCES = [
     [SHAPES["batch_t64"], SHAPES["verify_t2"]],
     [MoEShape("g300", 300, 1024, 16, 4, 256, 256), MoEShape("g96", 96, 1024, 16, 4, 256, 256)],
+    [MoEShape("w720", 720, 512, 64, 8, 896, 896), MoEShape("d24", 24, 1024, 16, 4, 256, 256)],
 ]
+SEQUENCE_PATHS = [["stream_bf16", "few_tokens"], ["stream_split", "stream_bf16"], ["wide", "decode"]]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("seq", range(len(SEQUENCES)))
 def test_noalloc_equals_moe_forward_on_consecutive_calls(seq):
+    import gpu_util as gu
     native.load()
+    assert [gu.layer_path(shape) for shape in SEQUENCES[seq]] == SEQUENCE_PATHS[seq]
     for i, shape in enumerate(SEQUENCES[seq]):
         (o_n, w_n, i_n), (o_f, w_f, i_f) = _both(shape, 8800 + 10 * seq + i)
         assert np.isfinite(o_n).all(), (shape.name, "non-finite output")
