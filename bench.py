@@ -25,8 +25,9 @@ I=768) it carries the metric's three parts:
     layer, one token per step, Markov routing) per step;
   * ``decode_t1`` and ``batch_t64``: the other decode configurations (one token
     of the small layer; 64 tokens with Zipf-skewed routing), each with its
-    dominant kernel against the HBM roofline, the layer-level selected-expert
-    GB/s and its own CPU baseline;
+    dominant kernel against the HBM roofline (the streaming GEMMs of the 64-token
+    layer over the whole layer step), the layer-level selected-expert GB/s and
+    its own CPU baseline;
 and the CPU baseline (the C restatement in oracle/, OpenMP, on this host) on a
 bounded sample of the default workload, with the single-threaded numpy
 oracle's rate beside it.
@@ -198,15 +199,16 @@ class Setup:
         self.xs = torch.randn((self.n_inputs, T, d), device=dev, generator=gen).to(torch.bfloat16)
         if hc:
             self.streams = torch.randn((self.n_inputs, T, hc, d), device=dev, generator=gen)
-        # the layer's routed gate/up kernel: token-major for a few tokens, tiled
-        # GEMV up to 64 tokens, grouped MFMA GEMMs beyond
-        # the token-major and decode kernels cover d / 512 in {2, 4, 6, 8} and
-        # I / 128 in {1, 2, 4, 6, 8, 16} chunks; other shapes run on the general
-        # GEMV kernels
-        self.decode_kernels = (d % 512 == 0 and d // 512 in (2, 4, 6, 8) and I % 128 == 0
-                               and I // 128 in (1, 2, 4, 6, 8, 16))
-        self.few_token = T <= 4 and k <= 8 and self.decode_kernels
-        self.grouped = T > 64
+        # the layer's routed gate/up kernel: token-major for a few tokens, decode
+        # kernels or streaming grouped GEMMs for decode batches, wide grouped
+        # GEMMs for prompts
+        path = self.lib.glm_moe_forward_path(T, d, E, k, I, Is, native.GLM_FMT_BF16, None, None,
+                                             None)
+        self.few_token = path == native.GLM_PATH_FEW_TOKENS
+        self.decode_kernels = path == native.GLM_PATH_DECODE
+        self.grouped = path == native.GLM_PATH_WIDE
+        # no entry point of its own: timed inside the layer step
+        self.streaming = path in (native.GLM_PATH_STREAM_BF16, native.GLM_PATH_STREAM_SPLIT)
         self.act_format = {"fp8x2": native.GLM_ACT_FP8X2, "fp6x2": native.GLM_ACT_FP6X2,
                            "fp4": native.GLM_ACT_FP4, "fp8fp6": native.GLM_ACT_FP8FP6}[
                                getattr(args, "act_format", "fp8x2")]
@@ -327,6 +329,8 @@ class Setup:
     def kernel_name(self) -> str:
         """The dominant kernel's instantiation, as rocprofv3 names it."""
         d, E = self.d, self.E
+        if self.streaming:
+            return "grouped_stream_kernel"
         if self.grouped:
             return f"grouped_f8f6f4_w8_kernel<2, {self.act_format}>"
         if self.few_token:
@@ -497,17 +501,24 @@ def measure(args, torch, np, workload: str, *, steps: int, warmup: int, traffic:
     tokens_per_s = T / (ms_per_step / 1e3)
 
     # ------------------------------------------------------------ dominant kernel
-    gk = capture(S.gate_up, 0, R)
-    gk.replay()
-    k_ms, _ = timed(gk, R)
-    bytes_per_launch = sum(S.kernel_bytes(r) for r in range(R)) / R
+    if S.streaming:
+        # the routed GEMMs run inside the layer only: their bound against the step
+        k_ms, R = ms_per_step, steps
+        bytes_per_launch = sum(unique_per_step) / steps * shape.expert_bytes
+    else:
+        gk = capture(S.gate_up, 0, R)
+        gk.replay()
+        k_ms, _ = timed(gk, R)
+        bytes_per_launch = sum(S.kernel_bytes(r) for r in range(R)) / R
+        del gk
     achieved = bytes_per_launch / (k_ms / 1e3) / 1e9
     tflops = S.kernel_flops() / (k_ms / 1e3) / 1e12
-    del gk
     torch.cuda.synchronize()
 
     traffic_v, traffic_note = None, "not measured (--traffic 0)"
-    if traffic:
+    if S.streaming:
+        traffic_note = "not measured (the kernel runs inside the layer only)"
+    elif traffic:
         traffic_v, traffic_note = measure_traffic(args, workload, S.kernel_name())
 
     cpu = None
@@ -619,8 +630,8 @@ def prefill_leg(r: dict, counters: dict | None) -> dict:
 
 def decode_leg(r: dict) -> dict:
     """A decode configuration's figures: the layer's tokens/s, the dominant
-    routed gate/up kernel against the HBM roofline (HIP events over a graph
-    of its launches), the selected experts' bytes over the layer step's device
+    routed kernel against the HBM roofline (HIP events over a graph of its
+    launches, or of the layer's), the selected experts' bytes over the layer step's device
     time, and the C restatement on this host's cores."""
     leg = {"workload": describe(r), "tokens_per_s": round(r["tokens_per_s"], 1),
            "ms_per_step": round(r["ms_per_step"], 5), "roofline": r["roofline"]}
@@ -654,6 +665,9 @@ def main() -> int:
         return dispatch_bench(args, torch, np)
     if args.mode == "kernel":
         S = Setup(args, torch, np, args.workload, args.steps, args.warmup, args.min_rotation_gb)
+        if S.streaming:
+            print(json.dumps({"error": "the streaming GEMMs run inside the layer only"}))
+            return 2
         S.kernel_plans(args.kernel_launches)
         for r in range(args.kernel_launches):
             S.gate_up(r)
@@ -732,7 +746,9 @@ def main() -> int:
 
 def roofline(S, achieved, tflops, bytes_per_launch, k_ms, R, traffic, traffic_note):
     """The dominant kernel against its bound: HBM for the decode GEMVs, the
-    dense MXFP4 MFMA peak for the grouped prefill GEMM."""
+    dense MXFP4 MFMA peak for the grouped prefill GEMM.  The streaming GEMMs,
+    which have no entry point of their own: all three routed projections' bytes
+    over the whole layer step."""
     common = {"traffic": traffic, "traffic_note": traffic_note,
               "bytes_per_launch": round(bytes_per_launch), "avg_launch_us": round(k_ms * 1e3, 3),
               "launches": R, "unique_experts_per_launch": round(sum(S.unique) / R, 2)}
@@ -751,6 +767,11 @@ def roofline(S, achieved, tflops, bytes_per_launch, k_ms, R, traffic, traffic_no
                 "design_ceiling": ceiling,
                 "frac_of_design_ceiling": round(tflops / ceiling, 4),
                 **common}
+    if S.streaming:
+        common["unique_experts_per_launch"] = round(bytes_per_launch / S.shape.expert_bytes, 2)
+        return {"kernel": S.kernel_name() + " (routed gate/up and down, over the whole layer step)",
+                "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS,
+                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4), **common}
     return {"kernel": S.kernel_name() + (" (few-token selection + routed MXFP4 gate/up + SwiGLU)"
                                          if S.few_token else
                                          " (routed MXFP4 gate/up + SwiGLU)"),
