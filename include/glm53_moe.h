@@ -94,7 +94,7 @@ int glm_router_topk(void *stream, const uint16_t *x, int T, int d, const float *
  * chunk sums the counts of the chunks before it and places its pairs
  * (pair_token holds the chunk counts until it is filled last; the result is
  * the same).
- * Limits: E <= 448 (one workgroup's LDS holds the per-expert bitmaps).
+ * Limits: E <= 448 (one workgroup's LDS holds the per-expert counts).
  */
 int glm_moe_dispatch(void *stream, const uint32_t *indices, int T, int top_k, int E,
                      int32_t *counts, int32_t *offsets, int32_t *perm, int32_t *inv,
@@ -373,7 +373,9 @@ int glm_moe_workspace_init(void *stream, void *workspace, size_t workspace_bytes
  * gate/up), top-k selection + routed gate/up (+ shared down), routed down +
  * weighted combine.  Up to 64 tokens (T*k <= 512) it is the decode path:
  * router logits, selection, dispatch (+ shared down), routed gate/up, routed
- * down, combine.  Beyond that the dispatch and the grouped MFMA GEMMs.
+ * down, combine; from 16 tokens on only for layers of few work items or few
+ * bytes.  Else the dispatch and the grouped MFMA GEMMs, streaming or wide
+ * (glm_moe_forward_path tells which kernels a call runs on).
  * shared_in (may be NULL): the shared expert's bf16 output [T][d] computed by
  * the caller -- e.g. with glm_dense_mlp on a second stream, overlapping the
  * routing -- in which case the shared weights are not read.

@@ -67,8 +67,8 @@ struct DenseTile {
 };
 
 // bf16 stages hold 64 of K: token tiles are pairs of blocks a wave there, so
-// that a stage is whole rounds of loads
-// and MXFP4's need 128 weight rows for that; gate/up tiles hold both projections.
+// that a stage is whole rounds of loads, and MXFP4's need 128 weight rows for
+// that; gate/up tiles hold both projections.
 // 64-row tiles (br 1) are for few tokens.
 template <int FMT, int NPROJ>
 constexpr bool dense_takes(int br, int tb) {
@@ -80,7 +80,8 @@ constexpr bool dense_takes(int br, int tb) {
 // A workgroup alone on its CU took, in us per 128 of K (MXFP8, K 4096):
 // 0.81 + 0.055 br tb with 256-row tiles (tb 1 / 2 / 3 / 4: 1.04 / 1.23 / 1.46 /
 // 1.68), 0.48 + 0.08 br tb with 128-row ones (0.65 / 0.78 / 0.93 / 1.15); the
-// weights below are these in one unit.  64-row tiles (tb 1 / 2: 0.43 / 0.52)
+// weights below are these in one unit, used for the other formats and for
+// gate/up as well.  64-row tiles (tb 1 / 2: 0.43 / 0.52)
 // where those would leave most of the chip idle: 100 tokens at N = K = 4096
 // 15.8 us in MXFP8 and 20.1 in bf16, where 128-row tiles take 20.5 and 26.3.
 // Picked against measured best at

@@ -129,7 +129,7 @@ __device__ __forceinline__ void dense_item(const DenseArgs &a, int lin) {
   const int f0 = rt * kFeat, t0 = tt * L::kTok;
 
   // ---- load assignment, fixed over the K loop: load j of wave w fills the
-  // (8 j + w)-th 1 KB of the tokens, then of the weight rows.  Tokens past the
+  // (kWaves j + w)-th 1 KB of the tokens, then of the weight rows.  Tokens past the
   // last one and rows past the last feature re-read the last (their MFMA rows
   // and columns are independent of the others and not stored).
   uint32_t xoff[L::kXLoads], woff[L::kWLoads];

@@ -1,5 +1,6 @@
 // Decode-size routed-MoE layer (T <= 64, T*k <= 512 pairs; from 16 tokens on
-// only small layers, see glm_grouped_stream_decode) in five kernels:
+// layers of few work items or few bytes, see glm_grouped_stream_decode) in five
+// kernels:
 //
 //   1. route_logits_kernel    router logits (one block per expert, 4 waves
 //                             split d) -- and, in extra blocks, the bf16
@@ -1022,10 +1023,11 @@ size_t glm_select_dispatch_lds_bytes(int EPL) {
 // Whether the decode kernels cover this layer shape: gate/up waves take d/512
 // chunks of 128 (d / 4 per wave), down waves the whole K = I in I/128 chunks
 // (16 at the real expert geometry, I 2048).  A wave's chunks are one batch of
-// loads whatever their count, so every count within the registers is taken;
-// a count left out puts the layer on the work-list GEMVs, or on one thread per
-// output where K has no split there: two layers of one token at d 3072, I 896
-// took 495 us (63 here), 23 tokens at d 2560, I 896 26.6 ms (94 us).
+// loads whatever their count, so odd counts are taken too: two layers of one
+// token at d 3072, I 896 took 495 us (63 here) and 23 tokens at d 2560, I 896
+// 26.6 ms (94 us) as one thread per output.  Down counts of 11 to 15 are left out:
+// 12 has a split on the work-list GEMVs; 11, 13, 14 and 15 have none there and run
+// one thread per output below 16 tokens, the streaming grouped GEMMs from 16 on.
 static bool gate_up_chunks_ok(int c) { return c >= 2 && c <= 8; }
 static bool down_chunks_ok(int c) { return (c >= 1 && c <= 10) || c == 16; }
 

@@ -215,9 +215,12 @@ bool glm_router_gemm_supported(int T, int d) {
 }
 
 // Up to 96 M products the f32 MFMA over 16-way K splits, which fills the chip
-// and needs no split of the weights, beats the bf16 form from 256 tokens on:
-// the layer at 333 tokens, d 2048, E 128 (87 M) takes 106.0 us instead of 110.4;
-// 200 tokens, d 4096, E 288 (236 M) take 17 us here, 1023 24.8 in the bf16 form.
+// and needs no split of the weights, beats the bf16 form behind its own weight
+// split from 256 tokens on.  Layer times, f32 against bf16 form (d, E, tokens): 1024,
+// 64, 256 (17 M) 30.4 : 33.6 us; 2048, 128, 256 (67 M) 87.5 : 92.8; 333 (87 M) 92.7 : 98.3;
+// 4096, 64, 384 (101 M) 80.7 : 89.0.  They cross between 150 and 200 M, later at fewer
+// experts: 2048, 128, 512 (134 M) 106.6 : 111.9, 640 (168 M) 118.9 : 118.3, 768 (201 M)
+// 135.9 : 123.8; 4096, 128, 400 (210 M) 113.3 : 121.9, 700 (367 M) 133.9 : 131.0.
 static bool router_f32_rule(int T, int d, int E) {
   return (long long)T * d * E <= 96LL << 20 && d % (32 * 16 * 2) == 0;
 }
